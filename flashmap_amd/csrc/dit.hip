@@ -156,35 +156,79 @@ __global__ __launch_bounds__(256) void noise_rows_kernel(const float *__restrict
 static bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
 // The several-jump draft's state over the vocabulary (flashmap/vllm/model.py:944-956,
-// 1031-1036): softmaxes over rows of up to ~10^5 fp32 values, one workgroup per row.
-// The row is read twice: once for its statistics (max and sum of exponentials, online
-// per thread, merged over the workgroup), once for the outputs (each thread re-reads the
-// 16-byte chunks it read the first time; a row is small enough to be served from the
-// cache the second time). Exponentials are expf; the division and the update use torch's
-// rounding points.
-constexpr int STATE_THREADS = 256;
+// 1031-1036): softmaxes over rows of up to ~10^5 values. A row goes to `parts` workgroups
+// (state_parts); each forms the whole row's statistics (max and sum of exponentials,
+// online per thread, merged over the workgroup) and writes its part of the outputs.
+//
+// Bound: HBM. Few rows are in flight (at most two 1024-thread workgroups per CU), so that
+// the second read of a row comes from the caches: with 256-thread workgroups each of 1024
+// rows was resident at once, 311 to 622 MB between the two reads. The arithmetic stays
+// below the stream: exponentials are exp_neg (9 issue slots against 18 for expf), the
+// divisions by a row's (or the call's) one divisor take its reciprocal once and three
+// operations per element (DivBy; 14 for an IEEE division). Measured, 1024 x 151936 (1.56
+// and 1.24 GB): update 422 -> 344 us with this arithmetic and these workgroups, 284 us with
+// the non-temporal second pass; embedding 400 -> 356 -> 284 us, 260 us with a quarter of the
+// row held (16 chunks held spill: 347 us). 512 threads per row: 312 and 266 us. In parts,
+// 64 rows: update 161 -> 42 us, embedding 155 -> 47 us; 16 rows: 123 -> 22, 111 -> 22 us.
+constexpr int STATE_THREADS = 1024;
+constexpr int STATE_CHUNKS = 4;  // 4-value chunks in flight per thread
+constexpr int STATE_HELD = 8;    // state_embed_rows: chunks per thread kept between the passes
 
-struct RowStats {
-  float m, s;  // max and sum of exp(x - m)
-};
-
-__device__ __forceinline__ RowStats merge_stats(RowStats a, RowStats b) {
-  const float m = fmaxf(a.m, b.m);
-  if (m == -INFINITY) return RowStats{m, 0.f};
-  const float sa = a.m == -INFINITY ? 0.f : __fmul_rn(a.s, expf(__fsub_rn(a.m, m)));
-  const float sb = b.m == -INFINITY ? 0.f : __fmul_rn(b.s, expf(__fsub_rn(b.m, m)));
-  return RowStats{m, __fadd_rn(sa, sb)};
+// exp(x) for x <= 0 (0 for -inf, NaN for NaN) to about an ulp: exp2 of the rounded x log2(e),
+// corrected by what that rounding left of x. r is NaN only for x = -inf (the result is 0
+// already) and NaN (the result is NaN): the max keeps it out of the product.
+__device__ __forceinline__ float exp_neg(float x) {
+  const float t = x * 1.44269504f;
+  const float p = __builtin_amdgcn_exp2f(t);
+  float r = __builtin_fmaf(-t, 0.693147182f, x);
+  r = __builtin_fmaf(-t, -1.90465421e-9f, r);
+  return __builtin_fmaf(p, fmaxf(r, -0.001f), p);
 }
 
-__device__ __forceinline__ void add_chunk(RowStats &st, const float (&x)[4]) {
-  const float mx = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));
-  if (mx == -INFINITY) return;  // nothing to add (and no exp(-inf - -inf))
-  if (mx > st.m) {
-    st.s = st.m == -INFINITY ? 0.f : __fmul_rn(st.s, expf(__fsub_rn(st.m, mx)));
-    st.m = mx;
+// a / c by c's reciprocal and one residual step: the rounded quotient but for rare
+// last-bit ties.
+struct DivBy {
+  float c, y;
+  __device__ __forceinline__ explicit DivBy(float c_) : c(c_), y(__fdiv_rn(1.0f, c_)) {}
+  __device__ __forceinline__ float operator()(float a) const {
+    const float q = a * y;
+    return __builtin_fmaf(__builtin_fmaf(-q, c, a), y, q);
   }
+  // The same where the quotient may be infinite (the residual is then NaN).
+  __device__ __forceinline__ float any(float a) const {
+    const float q = a * y, d = __builtin_fmaf(__builtin_fmaf(-q, c, a), y, q);
+    return d == d ? d : q;
+  }
+};
+
+// m starts at the lowest finite value, so that no difference below is inf - inf unless a
+// value is +inf (the row is then NaN, as torch has it).
+struct RowStats {
+  float m, s;  // max and sum of exp(x - m)
+  static __device__ __forceinline__ RowStats none() { return RowStats{-3.402823466e38f, 0.f}; }
+  __device__ __forceinline__ void raise(float mx) {
+    if (mx > m) {
+      s *= exp_neg(m - mx);
+      m = mx;
+    }
+  }
+  __device__ __forceinline__ void merge(const RowStats &o) {
+    const float mx = fmaxf(m, o.m);
+    s = s * exp_neg(m - mx) + o.s * exp_neg(o.m - mx);
+    m = mx;
+  }
+};
+
+template <int N>
+__device__ __forceinline__ void add_values(RowStats &st, const float (&x)[N]) {
+  float mx = x[0];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) st.s = __fadd_rn(st.s, expf(__fsub_rn(x[q], st.m)));
+  for (int q = 1; q < N; ++q) mx = fmaxf(mx, x[q]);
+  st.raise(mx);
+  float s = 0.f;
+#pragma unroll
+  for (int q = 0; q < N; ++q) s += exp_neg(x[q] - st.m);
+  st.s += s;
 }
 
 // The workgroup's statistics from each thread's.
@@ -192,20 +236,85 @@ __device__ __forceinline__ RowStats block_stats(RowStats st) {
   __shared__ RowStats part[STATE_THREADS / 64];
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) {
-    const RowStats other{__shfl_xor(st.m, o, 64), __shfl_xor(st.s, o, 64)};
-    st = merge_stats(st, other);
+    st.merge(RowStats{__shfl_xor(st.m, o, 64), __shfl_xor(st.s, o, 64)});
   }
   if ((threadIdx.x & 63) == 0) part[wave_id()] = st;
   __syncthreads();
   RowStats r = part[0];
 #pragma unroll
-  for (int w = 1; w < STATE_THREADS / 64; ++w) r = merge_stats(r, part[w]);
+  for (int w = 1; w < STATE_THREADS / 64; ++w) r.merge(part[w]);
   return r;
 }
 
+// Four consecutive values of a row of float or bf16.
+__device__ __forceinline__ f32x4_t load4(const float *p) { return *reinterpret_cast<const f32x4_t *>(p); }
+__device__ __forceinline__ f32x4_t load4(const uint16_t *p) {
+  const u32x2_t w = *reinterpret_cast<const u32x2_t *>(p);
+  return f32x4_t{bf16_lo(w[0]), bf16_hi(w[0]), bf16_lo(w[1]), bf16_hi(w[1])};
+}
+// Accesses of what the kernel does not touch again. NT: past the caches (non-temporal), so
+// that these keep the rows between their two reads; for outputs that would not stay in the
+// caches for the next kernel anyway (state_streams).
+template <bool NT>
+__device__ __forceinline__ f32x4_t load_last(const float *p) {
+  return NT ? __builtin_nontemporal_load(reinterpret_cast<const f32x4_t *>(p)) : load4(p);
+}
+template <bool NT, typename T, typename V>
+__device__ __forceinline__ void store_last(T *p, V v) {
+  if (NT)
+    __builtin_nontemporal_store(v, reinterpret_cast<V *>(p));
+  else
+    *reinterpret_cast<V *>(p) = v;
+}
+__device__ __forceinline__ float load1(const float *p) { return *p; }
+__device__ __forceinline__ float load1(const uint16_t *p) { return bf16_to_f32(*p); }
+
+// Adds scale * x over the 4-value chunks [from, end) of a row to this thread's statistics.
+template <typename T>
+__device__ __forceinline__ void add_chunks(RowStats &st, const T *x, int64_t from, int64_t end, float scale) {
+  int64_t c = from + threadIdx.x;
+  for (; c + (STATE_CHUNKS - 1) * STATE_THREADS < end; c += STATE_CHUNKS * STATE_THREADS) {
+    float e[4 * STATE_CHUNKS];
+#pragma unroll
+    for (int k = 0; k < STATE_CHUNKS; ++k) {
+      const f32x4_t v = load4(x + 4 * (c + k * STATE_THREADS));
+#pragma unroll
+      for (int q = 0; q < 4; ++q) e[4 * k + q] = v[q] * scale;
+    }
+    add_values(st, e);
+  }
+  for (; c < end; c += STATE_THREADS) {
+    const f32x4_t v = load4(x + 4 * c);
+    const float e[4] = {v[0] * scale, v[1] * scale, v[2] * scale, v[3] * scale};
+    add_values(st, e);
+  }
+}
+// ... over the values past a row's last whole chunk (vocab % 4 of them).
+template <typename T>
+__device__ __forceinline__ void add_tail(RowStats &st, const T *x, int64_t vocab, float scale) {
+  for (int64_t i = (vocab & ~3ll) + threadIdx.x; i < vocab; i += STATE_THREADS) {
+    const float e[1] = {load1(x + i) * scale};
+    add_values(st, e);
+  }
+}
+
+// This workgroup's part of a row of `chunks` 4-value chunks; the last part also takes the
+// values past them.
+struct PartOf {
+  int64_t first, end;
+  bool last;
+};
+__device__ __forceinline__ PartOf part_of(int64_t chunks) {
+  const uint32_t parts = gridDim.y, p = blockIdx.y;  // a power of two
+  const int sh = 31 - __builtin_clz(parts);
+  return PartOf{chunks * p >> sh, chunks * (p + 1) >> sh, p == parts - 1};
+}
+
 // POST: rows r < rows of out get bf16(softmax(evidence * state[r])) and rows rows + r
-// bf16(state[r]); otherwise out holds the state rows only (one read of the row).
-template <bool POST>
+// bf16(state[r]); otherwise out holds the state rows only (one read of the row). A
+// workgroup keeps the first STATE_HELD chunks per thread of its part in registers between
+// the two passes (32768 values); the rest is read again from the caches.
+template <bool POST, bool NT>
 __global__ __launch_bounds__(STATE_THREADS) void state_embed_rows_kernel(const float *__restrict__ state,
                                                                          int64_t vocab, int64_t ss, float evidence,
                                                                          uint16_t *__restrict__ out, int64_t os,
@@ -213,48 +322,57 @@ __global__ __launch_bounds__(STATE_THREADS) void state_embed_rows_kernel(const f
   const int64_t row = blockIdx.x;
   const float *x = state + row * ss;
   const int64_t chunks = vocab >> 2;
-  if constexpr (!POST) {
-    uint16_t *raw = out + row * os;
-#pragma unroll 4
-    for (int64_t c = threadIdx.x; c < chunks; c += STATE_THREADS) {
-      const f32x4_t v = *reinterpret_cast<const f32x4_t *>(x + 4 * c);
-      *reinterpret_cast<u32x2_t *>(raw + 4 * c) = u32x2_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-    }
-    for (int64_t i = 4 * chunks + threadIdx.x; i < vocab; i += STATE_THREADS)
-      raw[i] = (uint16_t)(pack_bf16x2(x[i], 0.f) & 0xffffu);
-    return;
-  }
-  RowStats st{-INFINITY, 0.f};
-#pragma unroll 4
-  for (int64_t c = threadIdx.x; c < chunks; c += STATE_THREADS) {
-    const f32x4_t v = *reinterpret_cast<const f32x4_t *>(x + 4 * c);
-    const float e[4] = {__fmul_rn(v[0], evidence), __fmul_rn(v[1], evidence), __fmul_rn(v[2], evidence),
-                        __fmul_rn(v[3], evidence)};
-    add_chunk(st, e);
-  }
-  for (int64_t i = 4 * chunks + threadIdx.x; i < vocab; i += STATE_THREADS) {  // the tail (vocab % 4)
-    const float e[4] = {__fmul_rn(x[i], evidence), -INFINITY, -INFINITY, -INFINITY};
-    add_chunk(st, e);
-  }
-  const RowStats t = block_stats(st);
-  uint16_t *post = out + row * os, *raw = out + (rows + row) * os;
-#pragma unroll 4
-  for (int64_t c = threadIdx.x; c < chunks; c += STATE_THREADS) {
-    const f32x4_t v = *reinterpret_cast<const f32x4_t *>(x + 4 * c);
-    float p[4];
+  uint16_t *post = out + row * os, *raw = POST ? out + (rows + row) * os : post;
+  const PartOf part = part_of(chunks);
+  RowStats t{0.f, 1.f};
+  f32x4_t held[STATE_HELD];
+  int64_t c = part.first + threadIdx.x;
+  if constexpr (POST) {
+    t = RowStats::none();
 #pragma unroll
-    for (int q = 0; q < 4; ++q) p[q] = __fdiv_rn(expf(__fsub_rn(__fmul_rn(v[q], evidence), t.m)), t.s);
-    *reinterpret_cast<u32x2_t *>(post + 4 * c) = u32x2_t{pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3])};
-    *reinterpret_cast<u32x2_t *>(raw + 4 * c) = u32x2_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+    for (int k = 0; k < STATE_HELD; ++k)
+      held[k] = c + k * STATE_THREADS < part.end ? load4(x + 4 * (c + k * STATE_THREADS)) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < STATE_HELD; ++k) {
+      if (c + k * STATE_THREADS < part.end) {
+        const float e[4] = {held[k][0] * evidence, held[k][1] * evidence, held[k][2] * evidence,
+                            held[k][3] * evidence};
+        add_values(t, e);
+      }
+    }
+    const int64_t next = part.first + STATE_HELD * STATE_THREADS;
+    add_chunks(t, x, 0, part.first, evidence);
+    add_chunks(t, x, next < part.end ? next : part.end, chunks, evidence);
+    add_tail(t, x, vocab, evidence);
+    t = block_stats(t);
   }
+  const DivBy div(t.s);
+  auto put = [&](int64_t c, f32x4_t v) {
+    if constexpr (POST) {
+      float p[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) p[q] = div(exp_neg(v[q] * evidence - t.m));
+      store_last<NT>(post + 4 * c, u32x2_t{pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3])});
+    }
+    store_last<NT>(raw + 4 * c, u32x2_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])});
+  };
+  if constexpr (POST) {
+#pragma unroll
+    for (int k = 0; k < STATE_HELD; ++k, c += STATE_THREADS)
+      if (c < part.end) put(c, held[k]);
+  }
+#pragma unroll 4
+  for (; c < part.end; c += STATE_THREADS) put(c, load_last<NT>(x + 4 * c));
+  if (!part.last) return;
   for (int64_t i = 4 * chunks + threadIdx.x; i < vocab; i += STATE_THREADS) {
-    const float p = __fdiv_rn(expf(__fsub_rn(__fmul_rn(x[i], evidence), t.m)), t.s);
-    post[i] = (uint16_t)(pack_bf16x2(p, 0.f) & 0xffffu);
+    if constexpr (POST)
+      post[i] = (uint16_t)(pack_bf16x2(div(exp_neg(x[i] * evidence - t.m)), 0.f) & 0xffffu);
     raw[i] = (uint16_t)(pack_bf16x2(x[i], 0.f) & 0xffffu);
   }
 }
 
 // state[r] = (c_keep * state[r] + c_new * softmax(logits[r])) / c_div in place, logits bf16.
+template <bool NT>
 __global__ __launch_bounds__(STATE_THREADS) void state_update_kernel(float *__restrict__ state, int64_t vocab,
                                                                      int64_t ss, const uint16_t *__restrict__ logits,
                                                                      int64_t ls, float c_keep, float c_new,
@@ -263,34 +381,42 @@ __global__ __launch_bounds__(STATE_THREADS) void state_update_kernel(float *__re
   float *x = state + row * ss;
   const uint16_t *lg = logits + row * ls;
   const int64_t chunks = vocab >> 2;
-  RowStats st{-INFINITY, 0.f};
-#pragma unroll 4
-  for (int64_t c = threadIdx.x; c < chunks; c += STATE_THREADS) {
-    const u32x2_t w = *reinterpret_cast<const u32x2_t *>(lg + 4 * c);
-    const float e[4] = {bf16_lo(w[0]), bf16_hi(w[0]), bf16_lo(w[1]), bf16_hi(w[1])};
-    add_chunk(st, e);
-  }
-  for (int64_t i = 4 * chunks + threadIdx.x; i < vocab; i += STATE_THREADS) {
-    const float e[4] = {__uint_as_float((uint32_t)lg[i] << 16), -INFINITY, -INFINITY, -INFINITY};
-    add_chunk(st, e);
-  }
-  const RowStats t = block_stats(st);
+  const PartOf part = part_of(chunks);
+  RowStats t = RowStats::none();
+  add_chunks(t, lg, 0, chunks, 1.f);
+  add_tail(t, lg, vocab, 1.f);
+  t = block_stats(t);
+  const DivBy div(t.s), scale(c_div);
   auto upd = [&](float s, float l) {
-    const float d = __fdiv_rn(expf(__fsub_rn(l, t.m)), t.s);
-    return __fdiv_rn(__fadd_rn(__fmul_rn(c_keep, s), __fmul_rn(c_new, d)), c_div);
+    return scale.any(c_keep * s + c_new * div(exp_neg(l - t.m)));
   };
 #pragma unroll 4
-  for (int64_t c = threadIdx.x; c < chunks; c += STATE_THREADS) {
-    const u32x2_t w = *reinterpret_cast<const u32x2_t *>(lg + 4 * c);
-    f32x4_t v = *reinterpret_cast<const f32x4_t *>(x + 4 * c);
-    v[0] = upd(v[0], bf16_lo(w[0]));
-    v[1] = upd(v[1], bf16_hi(w[0]));
-    v[2] = upd(v[2], bf16_lo(w[1]));
-    v[3] = upd(v[3], bf16_hi(w[1]));
-    *reinterpret_cast<f32x4_t *>(x + 4 * c) = v;
+  for (int64_t c = part.first + threadIdx.x; c < part.end; c += STATE_THREADS) {
+    const int64_t at = 4 * c;
+    const f32x4_t l = load4(lg + at);
+    f32x4_t v = load_last<NT>(x + at);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = upd(v[q], l[q]);
+    store_last<NT>(x + at, v);
   }
-  for (int64_t i = 4 * chunks + threadIdx.x; i < vocab; i += STATE_THREADS)
-    x[i] = upd(x[i], __uint_as_float((uint32_t)lg[i] << 16));
+  if (!part.last) return;
+  for (int64_t i = 4 * chunks + threadIdx.x; i < vocab; i += STATE_THREADS) x[i] = upd(x[i], load1(lg + i));
+}
+
+// Whether a call's state rows outgrow the 256 MB of the last cache level. Below that the
+// kernels' outputs are found there by whoever reads them next, and the non-temporal
+// accesses only cost: the state rows alone at 256 x 151936 (156 MB) 33 us, 42 us with them.
+static bool state_streams(int64_t rows, int64_t vocab) { return rows * vocab > (64ll << 20); }
+
+// Workgroups per row, a power of two: with fewer rows than two per CU the rest of the chip
+// takes parts of them, each part reading the whole row for its statistics again (from the
+// caches).
+static unsigned state_parts(int64_t rows) {
+  DeviceInfo info;
+  if (device_info(&info) != FM_OK) return 1;
+  unsigned p = 1;
+  while (p < 8 && 2 * p * rows <= 2 * (int64_t)info.cus) p *= 2;
+  return p;
 }
 
 }  // namespace fm
@@ -380,13 +506,12 @@ extern "C" int fm_state_embed_rows(const float *state, int64_t rows, int64_t voc
              "state must be 16-byte aligned with a row stride that is a multiple of 4 covering a row");
   FM_REQUIRE(((uintptr_t)out & 7) == 0 && out_stride % 4 == 0 && out_stride >= vocab,
              "out must be 8-byte aligned with a row stride that is a multiple of 4 covering a row");
-  const dim3 grid((unsigned)rows), block(STATE_THREADS);
-  if (posterior)
-    state_embed_rows_kernel<true><<<grid, block, 0, (hipStream_t)stream>>>(state, vocab, state_stride, evidence,
-                                                                           (uint16_t *)out, out_stride, rows);
-  else
-    state_embed_rows_kernel<false><<<grid, block, 0, (hipStream_t)stream>>>(state, vocab, state_stride, evidence,
-                                                                            (uint16_t *)out, out_stride, rows);
+  const dim3 grid((unsigned)rows, posterior ? state_parts(rows) : 1u), block(STATE_THREADS);
+  const bool nt = state_streams(rows, vocab);
+  auto *kernel = posterior ? (nt ? state_embed_rows_kernel<true, true> : state_embed_rows_kernel<true, false>)
+                           : (nt ? state_embed_rows_kernel<false, true> : state_embed_rows_kernel<false, false>);
+  kernel<<<grid, block, 0, (hipStream_t)stream>>>(state, vocab, state_stride, evidence, (uint16_t *)out, out_stride,
+                                                  rows);
   FM_CHECK_HIP(hipGetLastError());
   return FM_OK;
 }
@@ -406,7 +531,8 @@ extern "C" int fm_state_update(float *state, int64_t rows, int64_t vocab, int64_
   // The scalars as torch takes Python floats into a float32 op: computed in double, then
   // rounded to float.
   const float c_keep = (float)(1.0 - end), c_new = (float)(end - start), c_div = (float)(1.0 - start);
-  state_update_kernel<<<dim3((unsigned)rows), dim3(STATE_THREADS), 0, (hipStream_t)stream>>>(
+  auto *kernel = state_streams(rows, vocab) ? state_update_kernel<true> : state_update_kernel<false>;
+  kernel<<<dim3((unsigned)rows, state_parts(rows)), dim3(STATE_THREADS), 0, (hipStream_t)stream>>>(
       state, vocab, state_stride, (const uint16_t *)logits, logits_stride, c_keep, c_new, c_div);
   FM_CHECK_HIP(hipGetLastError());
   return FM_OK;

@@ -95,3 +95,38 @@ def test_state_wrapper_checks(dev):
         ops.state_update(torch.zeros(2, 8, device=dev), torch.zeros(2, 8, dtype=torch.bfloat16, device=dev), 1.0, 1.0)
     with pytest.raises(ValueError, match="logits must be bf16"):
         ops.state_update(torch.zeros(2, 8, device=dev), torch.zeros(2, 8, device=dev), 0.0, 0.5)
+
+
+# rows: 1 and 3 take eight workgroups a row, 200 two, 300 one; vocab: less than a chunk per
+# thread, around the 32768 values a workgroup keeps in registers and the chunks of a step,
+# remainders of 1 to 3; the last case is past the size whose accesses are non-temporal.
+@pytest.mark.parametrize("rows,vocab", [(r, v) for r in (1, 3, 200, 300)
+                                        for v in (1, 5, 4099, 32767, 32770, 49156)] + [(520, 131075)])
+def test_state_kernels_edges(dev, rows, vocab):
+    """Masked values (-inf, the lowest finite value), +inf and NaN as torch's softmax takes
+    them, and the sizes where a row's workgroups and passes change."""
+    print(f"state edges rows={rows} vocab={vocab}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(rows * 100003 + vocab)
+    state = _rows(torch.randn(rows, vocab, generator=g, device=dev), dev)
+    logits = _rows(2 * torch.randn(rows, vocab, generator=g, device=dev, dtype=torch.bfloat16), dev)
+    lowest = torch.finfo(torch.bfloat16).min
+    for t in (state, logits):
+        t[0, ::2] = -torch.inf if vocab > 1 else 0.0
+        if rows > 1:
+            t[1] = lowest
+        if rows > 2:
+            t[2] = -torch.inf
+        if rows > 4:
+            t[3, vocab // 2], t[4, vocab - 1] = torch.inf, torch.nan
+    before = state.double()
+    post = torch.softmax((1.5 * state).double(), -1)
+    both = ops.state_embed_rows(state, 1.5)
+    # float32 exponentials and sums to about 1e-6, then bf16: an ulp is 2^-8 of the value
+    assert torch.allclose(both[:rows].double(), post, rtol=2.0 ** -8, atol=1e-37, equal_nan=True)
+    assert torch.equal(both[rows:].view(torch.int16), state.bfloat16().view(torch.int16))
+    want = (0.4 * before + 0.3 * torch.softmax(logits.double(), -1)) / 0.7
+    out = ops.state_update(state, logits, 0.3, 0.6).double()
+    big = want.abs() > 1e38  # beyond float32 on the way to the quotient
+    assert torch.allclose(torch.where(big, 0.0, out), torch.where(big, 0.0, want), rtol=2e-5, atol=2e-6,
+                          equal_nan=True)
+    assert torch.equal(out[big].sign(), want[big].sign())
