@@ -71,6 +71,63 @@ def test_sample_rows(dev):
     assert (got[~gr] != x.float().argmax(1).numpy()[~gr]).mean() > 0.5
 
 
+def _all_keys(x, temps, seed, row0=0):
+    """Every logit's key, none skipped."""
+    return S.sample_keys(x.float().numpy(), temps.numpy(), np.zeros(len(x), dtype=bool), seed, row0=row0)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("rows,vocab,stride", [(1, 1, 1), (2, 7, 8), (3, 100, 100), (5, 8191, 8192), (4, 8193, 8200),
+                                               (3, 24581, 24581), (150, 49153, 49160)])
+def test_sample_rows_skips_only_losers(dev, dtype, rows, vocab, stride):
+    """Rows whose logits are flat (every one can win), peaked, far from zero, mostly -inf or
+    steps of about the bound (17 T), at temperatures on both sides of its range: each
+    sampled token is the one that the noise of every logit selects."""
+    g = gen(rows + vocab)
+    x = torch.randn(rows, stride, generator=g)
+    temps = 0.3 + torch.rand(rows, generator=g)
+    kinds = torch.arange(rows) % 6
+    x[kinds == 0] *= 0.1
+    x[kinds == 1, :1] += 30.0
+    x[kinds == 2] = x[kinds == 2] * 3 - 1000.0
+    x[kinds == 3] = torch.where(x[kinds == 3] > 1.0, x[kinds == 3], -float("inf"))
+    steps = torch.randint(0, 3, (int((kinds == 4).sum()), stride), generator=g)
+    x[kinds == 4] = 17.0 * temps[kinds == 4, None] * steps
+    temps[kinds == 5] = 50.0
+    x = x.to(dtype)[:, :vocab]
+    seed = 0x9_8765_4321
+    got = ops.sample_rows(x.to(dev), temps.to(dev), torch.zeros(rows, dtype=torch.bool, device=dev),
+                          torch.tensor(seed, device=dev)).cpu().numpy()
+    keys = _all_keys(x, temps, seed)
+    # A key rounds to float32 twice and its logs are within about two ulps each: the
+    # winner's key lies that close to the largest of all.
+    won = keys[np.arange(rows), got]
+    best = keys.max(axis=1)
+    slack = 1e-5 + 4 * 2.0 ** -23 * np.where(np.isfinite(best), np.abs(best), 0)
+    assert ((won >= best - slack) | (won == best)).all()
+
+
+def test_sample_rows_special_rows(dev):
+    vocab = 30000
+    x = torch.randn(6, vocab).bfloat16()
+    x[0] = -float("inf")  # every key -inf: the first index
+    x[1, 20000] = float("nan")
+    x[1, 29999] = float("nan")
+    x[2, 12345] = float("inf")
+    temps = torch.tensor([1.0, 1.0, 1.0, 1e-35, 1e35, 1.0])  # rows 3, 4: outside the bound's range
+    x[3, 777] = 20.0  # over 1e-35: +inf is the largest key and the first of them wins
+    x[3, :777] = -1.0
+    x[3, 778:] = -1.0
+    greedy = torch.zeros(6, dtype=torch.bool)
+    greedy[5] = True
+    seed = torch.tensor(5, dtype=torch.int64)
+    got = ops.sample_rows(x.to(dev), temps.to(dev), greedy.to(dev), seed.to(dev)).cpu()
+    assert got[:4].tolist() == [0, 20000, 12345, 777]
+    keys = _all_keys(x[4:5], temps[4:5], 5, row0=4)  # logit / T of about 0: the noise alone
+    assert int(got[4]) == int(keys[0].argmax())
+    assert int(got[5]) == int(x[5].float().argmax())
+
+
 def test_sample_rows_offsets_wrap_past_int32(dev):
     """row * V + col passes 2^31 for the last rows: int32 arithmetic, as the reference's."""
     rows, vocab = 300, 7_300_000
