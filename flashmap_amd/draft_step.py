@@ -248,16 +248,16 @@ class DraftStep:
         for i, layer in enumerate(model.layers):
             (_, _, g_self), (c_scale, c_shift, g_cross), (m_scale, m_shift, g_mlp) = mods[i]
             self_qn, self_kn, cross_qn = self.norms[i]
-            attn = ops.block_self_attention(F.linear(h, self.self_qkv[i]).view(batch, k, 3, heads, hd),
+            attn = ops.block_self_attention(ops.linear(h, self.self_qkv[i]).view(batch, k, 3, heads, hd),
                                             self_qn, self_kn, self.rope, slot_positions, layer.self_attn.q_norm.eps)
-            y = F.linear(attn.view(tokens, self.dim), layer.self_attn.o_proj.weight)
+            y = ops.linear(attn.view(tokens, self.dim), layer.self_attn.o_proj.weight)
             hidden, h = ops.adaln_residual(hidden, y, g_self, (c_scale, c_shift), layer.cross_attn_adaln.eps,
                                            x_out=hidden)
-            query = F.linear(h, layer.cross_attn.q_proj.weight).view(tokens, heads, hd)
+            query = ops.linear(h, layer.cross_attn.q_proj.weight).view(tokens, heads, hd)
             prologue = ops.Prologue(cross_qn, self.rope, slot_positions, layer.cross_attn.q_norm.eps)
             ctx = ops.block_attention_paged(query, caches[i], cu, seqused_k, block_table, k, self.max_model_len,
                                             self.scale, prologue=prologue, plan=plan)
-            y = F.linear(ctx.view(tokens, self.dim), layer.cross_attn.o_proj.weight)
+            y = ops.linear(ctx.view(tokens, self.dim), layer.cross_attn.o_proj.weight)
             hidden, h = ops.adaln_residual(hidden, y, g_cross, (m_scale, m_shift), layer.mlp_adaln.eps, x_out=hidden)
             y = layer.mlp(h)
             if i + 1 < len(model.layers):

@@ -148,6 +148,15 @@ class _Joined:
 # --------------------------------------------------------------------------- modules
 
 
+class _Linear(nn.Linear):
+    """``nn.Linear`` whose few-row calls run the framework's kernel (:func:`ops.linear`)."""
+
+    def forward(self, x: torch.Tensor) -> torch.Tensor:
+        if x.numel() > ops.LINEAR_ROWS * self.in_features:
+            return F.linear(x, self.weight, self.bias)
+        return ops.linear(x, self.weight, self.bias)
+
+
 class FlashMapRMSNorm(nn.Module):
     """RMSNorm whose scale ``weight / rms(x)`` is rounded to ``x``'s dtype before the
     multiply (flashmap/modeling_flashmap.py:69-80). As the q/k norm of an attention its
@@ -179,8 +188,8 @@ class FlashMapTimeEmbedding(nn.Module):
     def __init__(self, config):
         super().__init__()
         self.dim, self.scale = config.time_embed_dim, config.time_scale
-        self.linear_1 = nn.Linear(config.time_embed_dim, config.cond_dim)
-        self.linear_2 = nn.Linear(config.cond_dim, config.cond_dim)
+        self.linear_1 = _Linear(config.time_embed_dim, config.cond_dim)
+        self.linear_2 = _Linear(config.cond_dim, config.cond_dim)
 
     def forward(self, t: torch.Tensor) -> torch.Tensor:
         feats = _time_features(t, self.dim, self.scale).to(self.linear_1.weight.dtype)
@@ -195,7 +204,7 @@ class FlashMapAdaLayerNorm(nn.Module):
 
     def __init__(self, config):
         super().__init__()
-        self.linear = nn.Linear(config.cond_dim, 3 * config.hidden_size)
+        self.linear = _Linear(config.cond_dim, 3 * config.hidden_size)
         self.eps = config.layer_norm_eps
 
     def modulation(self, cond: torch.Tensor):
@@ -227,10 +236,10 @@ class FlashMapAttention(nn.Module):
         dim = config.hidden_size
         self.num_heads = config.num_attention_heads
         self.head_dim = dim // self.num_heads
-        self.q_proj = nn.Linear(dim, dim, bias=False)
-        self.k_proj = nn.Linear(dim, dim, bias=False)
-        self.v_proj = nn.Linear(dim, dim, bias=False)
-        self.o_proj = nn.Linear(dim, dim, bias=False)
+        self.q_proj = _Linear(dim, dim, bias=False)
+        self.k_proj = _Linear(dim, dim, bias=False)
+        self.v_proj = _Linear(dim, dim, bias=False)
+        self.o_proj = _Linear(dim, dim, bias=False)
         self.q_norm = FlashMapRMSNorm(self.head_dim, config.qk_norm_eps)
         self.k_norm = FlashMapRMSNorm(self.head_dim, config.qk_norm_eps)
         self._qkv = _Joined()
@@ -258,7 +267,8 @@ class FlashMapAttention(nn.Module):
             return self(x, rope, *self.project_kv(x, rope))
         if self.q_norm.eps != self.k_norm.eps:
             raise ValueError("the fused block attention takes one eps for the q and k norms")
-        qkv = F.linear(x, self._qkv((self.q_proj.weight, self.k_proj.weight, self.v_proj.weight)))
+        project = F.linear if b * t > ops.LINEAR_ROWS else ops.linear
+        qkv = project(x, self._qkv((self.q_proj.weight, self.k_proj.weight, self.v_proj.weight)))
         qkv = qkv.view(b, t, 3, self.num_heads, self.head_dim)
         out = ops.block_self_attention(qkv, self.q_norm.weight, self.k_norm.weight, _token_rope(rope, b, t), None,
                                        self.q_norm.eps)
@@ -274,11 +284,11 @@ class FlashMapMLP(nn.Module):
         self.mlp_type = getattr(config, "mlp_type", "gelu")
         dim, hidden = config.hidden_size, config.intermediate_size
         if self.mlp_type == "swiglu":
-            self.gate_up_proj = nn.Linear(dim, 2 * hidden, bias=False)
-            self.down_proj = nn.Linear(hidden, dim, bias=False)
+            self.gate_up_proj = _Linear(dim, 2 * hidden, bias=False)
+            self.down_proj = _Linear(hidden, dim, bias=False)
         else:
-            self.fc1 = nn.Linear(dim, hidden)
-            self.fc2 = nn.Linear(hidden, dim)
+            self.fc1 = _Linear(dim, hidden)
+            self.fc2 = _Linear(hidden, dim)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self.mlp_type != "swiglu":
@@ -471,21 +481,21 @@ class FlashMapDraftModel(nn.Module):
         dim, target_dim = cfg.hidden_size, cfg.target_hidden_size
         self.head_dim = dim // cfg.num_attention_heads
         # context features: the target's hidden states at target_layer_ids, and the anchor
-        self.fc = nn.Linear(len(cfg.target_layer_ids) * target_dim, dim, bias=False)
+        self.fc = _Linear(len(cfg.target_layer_ids) * target_dim, dim, bias=False)
         self.hidden_norm = FlashMapRMSNorm(dim, cfg.rms_norm_eps)
-        self.anchor_proj = nn.Linear(target_dim, dim)
+        self.anchor_proj = _Linear(target_dim, dim)
         self.anchor_norm = FlashMapRMSNorm(dim, cfg.rms_norm_eps)
         # state featurization
         self.state_norm = FlashMapRMSNorm(target_dim, cfg.rms_norm_eps)
         self.noise_norm = FlashMapRMSNorm(target_dim, cfg.rms_norm_eps)
         self.noise_gate = nn.Parameter(torch.ones(1))
         # the DiT
-        self.x_embed = nn.Linear(target_dim, dim)
+        self.x_embed = _Linear(target_dim, dim)
         self.time_embed = FlashMapTimeEmbedding(cfg)
         self.jump_embed = FlashMapTimeEmbedding(cfg)
         self.layers = nn.ModuleList(FlashMapLayer(cfg) for _ in range(cfg.num_hidden_layers))
         self.final_adaln = FlashMapAdaLayerNorm(cfg)
-        self.head = nn.Linear(dim, target_dim)
+        self.head = _Linear(dim, target_dim)
         if cfg.state_vocab_size is not None:
             self.register_buffer("draft_ids", torch.arange(cfg.state_vocab_size))
         self._kv_weight, self._k_norms = _Joined(), _Joined()

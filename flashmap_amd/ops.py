@@ -1206,6 +1206,73 @@ def adaln_residual(
     return x_out, h
 
 
+LINEAR_ROWS = 32  # the most rows fm_linear_rows takes
+
+
+def _linear_streams(rows: int, n: int, k: int) -> bool:
+    """Whether fm_linear_rows is the faster one: sixteen rows of it read no more than the
+    weights do, and past them (or long reductions, or the wide heads) the rows that every
+    workgroup reads again cost more than the library's tiling. Measured, us, this kernel
+    and the library's, weights from HBM: 16 rows, n x k 2048 x 2048 7.0 / 10.7, 6144 x 2048
+    11.7 / 12.2, 8192 x 2048 12.3 / 12.7, 2048 x 4096 11.2 / 14.6, 2048 x 8192 19.7 / 12.9,
+    32000 x 4096 80 / 57; 32 rows, 2048 x 2048 9.5 / 10.9, 4096 x 2048 10.5 / 11.7, 6144 x
+    2048 16.5 / 12.3."""
+    if k % 32 or not 0 < n <= 8192:
+        return False
+    return (rows <= 16 and k <= 4096) or (rows <= LINEAR_ROWS and k <= 2048 and n <= 4096)
+
+
+def _eager_here(*tensors: torch.Tensor | None) -> bool:
+    """Whether a plain kernel launch is all that a call on these tensors asks for: CUDA
+    tensors, no gradient (backward or forward mode), and nothing that watches or rewrites
+    torch's calls (autocast, subclasses and modes, functorch's transforms, tracers)."""
+    given = [t for t in tensors if t is not None]
+    return (
+        all(t.is_cuda and type(t) in (torch.Tensor, torch.nn.Parameter) for t in given)
+        and not (torch.is_grad_enabled() and any(t.requires_grad for t in given))
+        and not torch.is_autocast_enabled("cuda")
+        and not torch.overrides.has_torch_function(given)
+        and torch._C._len_torch_dispatch_stack() == 0
+        and torch._C._functorch.peek_interpreter_stack() is None
+        and torch.autograd.forward_ad._current_level < 0
+        and not torch.jit.is_tracing()
+        and not torch.compiler.is_compiling()
+    )
+
+
+def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
+    """``F.linear``. Few bf16 rows, which only stream the weights (``_linear_streams``),
+    run the framework's kernel (fm_linear_rows); the rest, and calls that ask for more than
+    a launch (``_eager_here``), torch's."""
+    k = weight.shape[-1]
+    if not x.is_cuda or x.numel() > LINEAR_ROWS * k:  # most calls: no further looks
+        return torch.nn.functional.linear(x, weight, bias)
+    rows = x.numel() // k if k else 0
+    if (
+        rows > 0
+        and weight.dim() == 2
+        and _linear_streams(rows, weight.shape[0], k)
+        and x.shape[-1] == k
+        and x.dtype == weight.dtype == torch.bfloat16
+        and (bias is None or (bias.dtype == torch.bfloat16 and bias.is_contiguous() and bias.shape == weight.shape[:1]))
+        and x.is_contiguous()
+        and weight.stride(1) == 1
+        and weight.stride(0) % 8 == 0
+        and weight.stride(0) >= k
+        and _eager_here(x, weight, bias)
+        and x.device == weight.device == (x.device if bias is None else bias.device)
+        and x.device.index == torch.cuda.current_device()
+        and x.data_ptr() % 16 == 0
+        and weight.data_ptr() % 16 == 0
+    ):
+        n = weight.shape[0]
+        out = torch.empty(*x.shape[:-1], n, dtype=torch.bfloat16, device=x.device)
+        call("fm_linear_rows", x.data_ptr(), k, weight.data_ptr(), weight.stride(0), _ptr(bias), out.data_ptr(), n,
+             rows, n, k, _stream(x))
+        return out
+    return torch.nn.functional.linear(x, weight, bias)
+
+
 def noise_rows(z: torch.Tensor, eigvals: torch.Tensor, eps: float, gain: float,
                z_bf16: torch.Tensor | None = None) -> tuple[torch.Tensor, torch.Tensor]:
     """The folded noise read-out's row pass (flashmap/vllm/model.py:915-925): for ``z

@@ -431,6 +431,15 @@ int fm_adaln_residual(const void *x, int64_t x_stride, const void *y, int64_t y_
                       void *x_out, int64_t x_out_stride, void *h_out, int64_t h_out_stride,
                       int64_t rows, int32_t dim, float eps, void *stream);
 
+/* The DiT's projections for the few rows of a lightly loaded step (the torch Linears of
+ * flashmap/modeling_flashmap.py:118-192): out = x weight^T (+ bias in fp32), rounded to
+ * bf16 once. x (rows, k), weight (n, k), bias (n,) or NULL, out (rows, n), all bf16 with
+ * row strides in elements (x, weight: 16-byte aligned, strides multiples of 8). rows at
+ * most 32, k a multiple of 32. */
+int fm_linear_rows(const void *x, int64_t x_stride, const void *weight, int64_t w_stride,
+                   const void *bias, void *out, int64_t out_stride, int32_t rows, int32_t n,
+                   int32_t k, void *stream);
+
 /* The row pass of the one-jump draft's folded noise read-out (flashmap/vllm/model.py:
  * 915-925 with the folds of flashmap/vllm/fold.py:45-75): for z (rows, hidden) fp32 with a
  * row stride, scale[r] = bf16(gain * rsqrt(sum_i z[r,i]^2 eigvals[i] + eps)) (bf16, rows)
