@@ -17,7 +17,7 @@
 // with 16-byte loads, keys it in registers and reduces (key, index) over the wavefront and
 // then the workgroup; a one-wavefront-per-row pass merges the tiles. The sampler: one
 // workgroup per (part of a row, row), which draws the noise only where it can matter
-// (sample_parts_kernel); the same pass merges the parts. NaN counts as the largest key,
+// (sample_parts_kernel, sample_plan); the same pass merges the parts. NaN counts as the largest key,
 // the first NaN winning (torch.argmax's rule).
 #include <math.h>
 #include <stdint.h>
@@ -151,11 +151,7 @@ __global__ __launch_bounds__(SEL_THREADS) void select_tiles_kernel(const SelectA
   const char *src = a.logits + row * a.row_bytes;
   float bk = -INFINITY;
   int32_t bi = INT32_MAX;
-  auto visit = [&](int64_t col, float key) {
-    const bool take = key > bk || bi == INT32_MAX || (key != key && bk == bk);
-    bk = take ? key : bk;
-    bi = take ? (int32_t)col : bi;
-  };
+  auto visit = [&](int64_t col, float key) { visit_next(bk, bi, key, (int32_t)col); };
   const int64_t base = (int64_t)tile * SEL_TILE;
   constexpr int IT = SEL_TILE / (8 * SEL_THREADS);
   if (a.vec && base + SEL_TILE <= a.vocab) {  // a whole tile: every load in flight first
@@ -192,27 +188,30 @@ __global__ __launch_bounds__(SEL_THREADS) void select_tiles_kernel(const SelectA
 // logits that can still win: those within 16.64 T of the largest key that any thread of the
 // workgroup has seen (an LDS maximum that only rises; a late read of it only costs work). A
 // wavefront first draws for its 64 lanes' largest logits of the tile, which sets the
-// bound near the row's best at once, then for the rest that pass it, gathered from the
-// lanes into an LDS queue and taken 64 at a time. Keys, and so tokens, are those of every
-// logit's own noise: what is skipped is below the maximum by more than the bound's
-// rounding. The bound is no bound (-inf: nothing is skipped) for temperatures whose
-// product with it could over- or underflow.
+// bound near the tile's best at once, then for the rest that pass it, gathered from the
+// lanes into an LDS queue and taken 64 at a time; where most pass (flat logits), each lane
+// takes its own instead, read again from the caches. The uniform word alone rules most
+// of these out before the logarithms. Keys, and so tokens, are those of every logit's own
+// noise: what is skipped is below the maximum by more than the bound's rounding. The bound
+// is no bound (-inf: nothing is skipped) for temperatures whose product with it could over-
+// or underflow. Greedy rows look for the largest logit under the same kind of bound.
 //
 // How much is left depends on the logits and T: of 151936 normal logits with 24 likely ones
-// 1 % to 30 % for T from 0.6 to 1.2. Where every logit can win, the queue costs what the
-// logarithms spared by the early test in visit gain. Greedy rows look for the largest
-// logit under the same kind of bound. Measured on 1024 x 151936, us (every logit drawn for /
-// this kernel): half the rows greedy, T of 0.6 to 1.2: 204 / 122; all sampled at 0.6 328 / 74,
-// 0.9 328 / 115, 1.2 328 / 196; equal logits 327 / 325; all greedy 75 / 61. With 256-thread
-// workgroups and each wavefront's own first bound the case took 216 us: 71 % of the first
-// 2048 logits pass a bound set by themselves, 11 % of 32768.
+// 1 % to 30 % for T from 0.6 to 1.2. Measured on 1024 x 151936 bf16, us (every logit drawn for
+// / this kernel): half the rows greedy, T of 0.6 to 1.2: 209 / 125; all sampled at 0.6 340 /
+// 83, 1.2 340 / 202; normal logits of sigma 1 331 / 329, equal logits 330 / 329; all greedy
+// 75 / 54. Rows that are not 16-byte aligned are read in whole granules all the same (RowView):
+// 1024 x 100003 half greedy 184 (logit by logit) / 89, all greedy 122 / 44.
 constexpr float GUMBEL_MAX = 16.64f;
-constexpr int SAMPLE_IT = 4;                             // 8-logit chunks per thread and step
+constexpr int SAMPLE_IT = 4;  // 8-logit chunks per thread of a tile
 constexpr int sample_tile(int threads) { return 8 * SAMPLE_IT * threads; }
+// More than this many of a wavefront's first 512 logits of a tile above the bound: past the
+// queue. 1024 x 151936, T = 1.2: 267 us at 256, 250 at 400, 252 without; equal logits 318, 318, 338.
+constexpr int SAMPLE_DIRECT = 400;
 constexpr int SAMPLE_QUEUE = 64 + 4 * 64;  // what a drain leaves and four logits of 64 lanes
 
 struct Pending {
-  int32_t col;
+  uint32_t col;
   float x;
 };
 
@@ -233,99 +232,154 @@ __device__ __forceinline__ float unordered(int32_t i) { return __int_as_float(i 
 // Eight consecutive logits as they are stored (few registers while a tile is in flight).
 template <int TY>
 struct Chunk {
-  u32x4_t w[TY == LOGITS_F32 ? 2 : 1];
+  static constexpr int WORDS = TY == LOGITS_F32 ? 8 : 4, PER_WORD = 8 / WORDS;
+  uint32_t w[WORDS];
   // The compiler takes the words as new from here on: the logits decoded before are not
   // kept for a later pass over them (32 registers, which would spill).
   __device__ __forceinline__ void forget() {
 #pragma unroll
-    for (int h = 0; h < (TY == LOGITS_F32 ? 2 : 1); ++h) asm volatile("" : "+v"(w[h]));
+    for (int q = 0; q < WORDS; ++q) asm volatile("" : "+v"(w[q]));
   }
   __device__ __forceinline__ float at(int j) const {
-    if (TY == LOGITS_F32) return __uint_as_float(w[j >> 2][j & 3]);
-    const uint32_t pair = w[0][j >> 1];
-    if (TY == LOGITS_BF16) return j & 1 ? bf16_hi(pair) : bf16_lo(pair);
-    return j & 1 ? f16_hi(pair) : f16_lo(pair);
+    const uint32_t v = w[j / PER_WORD];
+    if (TY == LOGITS_F32) return __uint_as_float(v);
+    if (TY == LOGITS_BF16) return j & 1 ? bf16_hi(v) : bf16_lo(v);
+    return j & 1 ? f16_hi(v) : f16_lo(v);
+  }
+  // -inf in the place of logit j.
+  __device__ __forceinline__ void drop(int j) {
+    uint32_t &v = w[j / PER_WORD];
+    if (TY == LOGITS_F32)
+      v = 0xFF800000u;
+    else
+      v = j & 1 ? (v & 0xFFFFu) | (TY == LOGITS_BF16 ? 0xFF800000u : 0xFC000000u)
+                : (v & 0xFFFF0000u) | (TY == LOGITS_BF16 ? 0xFF80u : 0xFC00u);
   }
 };
 
-// The chunk from col on, -inf past the vocabulary (which col itself may be).
+// A row as 16-byte granules from the one its first logit lies in: `skip` logits of that
+// granule come before the row, and the last granule may end past it. Loads are of whole
+// granules with a logit of the row in them (no allocation ends inside one); the logits
+// around the row are dropped after the load.
 template <int TY>
-__device__ __forceinline__ Chunk<TY> chunk_at(const SelectArgs &a, const char *src, int64_t col) {
-  constexpr int ES = TY == LOGITS_F32 ? 4 : 2;
-  Chunk<TY> c;
-  if (a.vec && col + 8 <= a.vocab) {
+struct RowView {
+  static constexpr int ES = TY == LOGITS_F32 ? 4 : 2;
+  const char *from;
+  uint32_t skip, vocab, last;  // last: the row's last granule
+  __device__ __forceinline__ RowView(const SelectArgs &a, int64_t row) {
+    const char *src = a.logits + row * a.row_bytes;
+    skip = (uint32_t)((uintptr_t)src & 15) / ES;
+    from = src - skip * ES;
+    vocab = (uint32_t)a.vocab;
+    last = (uint32_t)(((uint64_t)skip + vocab - 1) * ES / 16);
+  }
+  // Chunk g: the logits of columns 8 g - skip to 8 g - skip + 7.
+  __device__ __forceinline__ Chunk<TY> chunk(uint32_t g) const {
+    Chunk<TY> c;
 #pragma unroll
-    for (int h = 0; h < ES / 2; ++h) c.w[h] = load16(src + col * ES + 16 * h);
+    for (int h = 0; h < ES / 2; ++h) {
+      const uint32_t n = g * (ES / 2) + h;
+      const u32x4_t v = load16(from + 16 * (uint64_t)(n < last ? n : last));
+#pragma unroll
+      for (int q = 0; q < 4; ++q) c.w[4 * h + q] = v[q];
+    }
     return c;
   }
-#pragma unroll
-  for (int q = 0; q < 2 * ES; ++q) {
-    uint32_t w = 0;
-#pragma unroll
-    for (int h = 0; h < 4 / ES; ++h) {
-      const int64_t i = col + q * (4 / ES) + h;
-      const bool in = i < a.vocab;
-      if (TY == LOGITS_F32)
-        w = in ? reinterpret_cast<const uint32_t *>(src)[i] : 0xFF800000u;
-      else
-        w |= (in ? (uint32_t) reinterpret_cast<const uint16_t *>(src)[i] : TY == LOGITS_BF16 ? 0xFF80u : 0xFC00u) << (16 * h);
-    }
-    c.w[q >> 2][q & 3] = w;
+  // Whether some of n chunks from g on reach past either end.
+  __device__ __forceinline__ bool edge(uint32_t g, uint32_t n) const {
+    return (g == 0 && skip != 0) || 8 * ((uint64_t)g + n) > (uint64_t)skip + vocab;
   }
-  return c;
+  __device__ __forceinline__ void trim(Chunk<TY> &c, uint32_t g) const {
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (8 * g - skip + j >= vocab) c.drop(j);
+  }
+};
+
+// The largest of a thread's logits of a tile (NaN aside) and whether one is NaN.
+template <int TY>
+__device__ __forceinline__ float tile_max(Chunk<TY> (&x)[SAMPLE_IT], bool &nan) {
+  float m = -INFINITY;
+  nan = false;
+#pragma unroll
+  for (int it = 0; it < SAMPLE_IT; ++it) {
+#pragma unroll
+    for (int j = 0; j < 8; j += 2) {
+      const float p = x[it].at(j), q = x[it].at(j + 1);
+      m = fmaxf(m, fmaxf(p, q));
+      nan |= __builtin_isunordered(p, q);
+    }
+    x[it].forget();
+  }
+  return m;
 }
 
+__device__ __forceinline__ float sample_uniform(uint32_t offset, uint64_t seed) {
+  uint32_t c[4] = {offset, 0u, 0u, 0u};
+  philox4x32_10(c, (uint32_t)seed, (uint32_t)(seed >> 32));
+  return word_to_uniform(c[0]);
+}
+__device__ __forceinline__ float sample_key(float x, float temp, float u) { return x / temp - logf(-logf(u)); }
+
+// A row of at most a chunk per thread.
 template <int TY, int THREADS>
+__device__ __forceinline__ void sample_short(const SelectArgs &a, const RowView<TY> &view, int64_t row) {
+  const Chunk<TY> c = view.chunk(threadIdx.x);
+  const bool noisy = a.greedy[row] == 0;
+  const float temp = a.temps[row];
+  const uint64_t seed = (uint64_t)a.seed[0];
+  const uint32_t row_off = (uint32_t)row * view.vocab, col0 = 8 * threadIdx.x - view.skip;
+  float bk = -INFINITY;
+  int32_t bi = INT32_MAX;
+  if (8 * threadIdx.x < view.skip + view.vocab) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      float key = c.at(j);
+      if (noisy) key = sample_key(key, temp, sample_uniform(row_off + col0 + j, seed));
+      if (col0 + j < view.vocab) visit_next(bk, bi, key, (int32_t)(col0 + j));
+    }
+  }
+  store_best<THREADS>(a, row, blockIdx.x, bk, bi);
+}
+
+// SEVERAL: tiles per workgroup; else one.
+template <int TY, int THREADS, bool SEVERAL>
 __global__ __launch_bounds__(THREADS, TY == LOGITS_F32 ? 4 : 8) void sample_parts_kernel(const SelectArgs a) {
-  constexpr int TILE = sample_tile(THREADS), STEP = 8 * THREADS;  // STEP: columns between a thread's chunks
+  constexpr uint32_t CHUNKS = SAMPLE_IT * THREADS;  // of a tile
+  constexpr uint32_t STEP = 8 * THREADS;            // columns between a thread's chunks
   __shared__ Pending queues[THREADS / 64][SAMPLE_QUEUE];
   __shared__ int32_t bound;
   const int64_t row = blockIdx.y;
-  const char *src = a.logits + row * a.row_bytes;
-  // This thread's logits of the tile at base: columns col0 + it * STEP + j, the first
-  // `left` of which (counted from col0) the vocabulary holds.
-  const int64_t hop = (int64_t)gridDim.x * TILE;
-  auto load = [&](Chunk<TY>(&x)[SAMPLE_IT], int64_t base) {
+  const RowView<TY> view(a, row);
+  const uint32_t chunks = (view.skip + view.vocab + 7) / 8, hop = gridDim.x * CHUNKS;
+  if (!SEVERAL && chunks <= THREADS) {  // a chunk per thread: every logit drawn for, no bound
+    sample_short<TY, THREADS>(a, view, row);
+    return;
+  }
+  // This thread's logits of the tile of chunks from g on: columns col0_of(g) + it * STEP + j.
+  auto load = [&](Chunk<TY>(&x)[SAMPLE_IT], uint32_t g) {
 #pragma unroll
-    for (int it = 0; it < SAMPLE_IT; ++it) x[it] = chunk_at<TY>(a, src, base + it * STEP + 8 * (int)threadIdx.x);
+    for (int it = 0; it < SAMPLE_IT; ++it) x[it] = view.chunk(g + it * THREADS + threadIdx.x);
   };
-  auto left_of = [&](int64_t col0) { return (int32_t)(a.vocab - col0 < TILE ? a.vocab - col0 : TILE); };
+  auto trim = [&](Chunk<TY>(&x)[SAMPLE_IT], uint32_t g) {
+    if (!view.edge(g, CHUNKS)) return;
+#pragma unroll
+    for (int it = 0; it < SAMPLE_IT; ++it) view.trim(x[it], g + it * THREADS + threadIdx.x);
+  };
+  auto col0_of = [&](uint32_t g) { return 8 * (g + (uint32_t)threadIdx.x) - view.skip; };
   // The first tile is on its way before the row's own values are looked at.
-  const int64_t first = (int64_t)blockIdx.x * TILE;
+  const uint32_t first = blockIdx.x * CHUNKS;
   Chunk<TY> x[SAMPLE_IT];
   load(x, first);
   const bool noisy = a.greedy[row] == 0;
   const float temp = a.temps[row];
   const uint64_t seed = (uint64_t)a.seed[0];
-  const uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)(seed >> 32);
-  // int32 offsets row * V + col, as the reference's kernel forms them
-  const uint32_t row_off = (uint32_t)row * (uint32_t)a.vocab;
   if (threadIdx.x == 0) bound = ordered(-INFINITY);
-  __syncthreads();
+  if (SEVERAL || noisy) __syncthreads();
+  trim(x, first);
   float bk = -INFINITY;
   int32_t bi = INT32_MAX;
   const int lane = threadIdx.x & 63;
-  Pending *queue = queues[wave_id()];
-  int queued = 0;  // wave-uniform
-  const bool boundable = temp > 1e-30f && temp < 1e30f;
-  const float inv_temp = 1.f / temp;
-  float low = -INFINITY;   // logits below it cannot win
-  float need = -INFINITY;  // the bound less its slack (see visit)
-  auto uniform = [&](int32_t col) {
-    uint32_t c[4] = {row_off + (uint32_t)col, 0u, 0u, 0u};
-    philox4x32_10(c, k0, k1);
-    return word_to_uniform(c[0]);
-  };
-  auto keyed = [&](float x, float u) { return x / temp - logf(-logf(u)); };
-  // Visits come in any order here: the full order of keys and indices. A key of at least b
-  // has -log(u) <= exp(x / T - b), and 1 - u <= -log(u): past exp of the slack above it (2 %,
-  // and 2e-6 of b for the roundings), the word alone rules the logit out.
-  auto visit = [&](int32_t col, float x) {
-    const float u = uniform(col);
-    if (1.f - u > __builtin_amdgcn_exp2f((x * inv_temp - need) * 1.44269504f)) return;
-    const float key = keyed(x, u);
-    if (better(key, col, bk, bi)) bk = key, bi = col;
-  };
   auto raise = [&](float key) {  // the bound takes this wavefront's largest key (NaN aside)
     key = key == key ? key : -INFINITY;
 #pragma unroll
@@ -334,6 +388,59 @@ __global__ __launch_bounds__(THREADS, TY == LOGITS_F32 ? 4 : 8) void sample_part
     wave_lds_fence();
   };
   auto bound_now = [&] { return unordered(*(volatile __attribute__((address_space(3))) int32_t *)&bound); };
+  if (!noisy) {  // the largest logit: tiles without one that reaches the bound are passed over
+    Chunk<TY> next[SAMPLE_IT];  // SEVERAL: the next tile in flight
+    for (uint32_t g = first;;) {
+      if (SEVERAL && g + hop < chunks) load(next, g + hop);
+      bool nan;
+      const float m = tile_max<TY>(x, nan);
+      if (!SEVERAL || g == first || __ballot(!(m < bound_now()) || nan) != 0) {
+        const uint32_t col0 = col0_of(g);
+        if (__ballot(nan || m == -INFINITY) == 0) {
+          uint32_t at = 0;
+#pragma unroll
+          for (int it = SAMPLE_IT - 1; it >= 0; --it)
+#pragma unroll
+            for (int j = 7; j >= 0; --j) at = x[it].at(j) == m ? it * STEP + j : at;
+          visit_next(bk, bi, m, (int32_t)(col0 + at));
+        } else {
+#pragma unroll
+          for (int it = 0; it < SAMPLE_IT; ++it)
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+              if (col0 + it * STEP + j < view.vocab) visit_next(bk, bi, x[it].at(j), (int32_t)(col0 + it * STEP + j));
+        }
+        if (SEVERAL && g + hop < chunks) raise(bk);
+      }
+      g += hop;
+      if (!SEVERAL || g >= chunks) break;
+#pragma unroll
+      for (int it = 0; it < SAMPLE_IT; ++it) x[it] = next[it];
+      trim(x, g);
+    }
+    store_best<THREADS>(a, row, blockIdx.x, bk, bi);
+    return;
+  }
+  // int32 offsets row * V + col, as the reference's kernel forms them
+  const uint32_t row_off = (uint32_t)row * view.vocab;
+  Pending *queue = queues[wave_id()];
+  int queued = 0;  // wave-uniform
+  const bool boundable = temp > 1e-30f && temp < 1e30f;
+  const float inv_temp = 1.f / temp;
+  float low = -INFINITY;   // logits below it cannot win
+  float need = -INFINITY;  // the bound less its slack (see visit)
+  auto uniform = [&](uint32_t col) { return sample_uniform(row_off + col, seed); };
+  auto keyed = [&](float x, float u) { return sample_key(x, temp, u); };
+  // Visits come in any order here: the full order of keys and indices. A key of at least b
+  // has -log(u) <= exp(x / T - b), and 1 - u <= -log(u): past exp of the slack above it (2 %,
+  // and 2e-6 of b for the roundings), the word alone rules the logit out.
+  auto loses = [&](float x, float u) {
+    return 1.f - u > __builtin_amdgcn_exp2f((x * inv_temp - need) * 1.44269504f);
+  };
+  auto visit = [&](uint32_t col, float x, float u) {
+    const float key = keyed(x, u);
+    if (col < view.vocab && better(key, (int32_t)col, bk, bi)) bk = key, bi = (int32_t)col;
+  };
   auto lower = [&] {
     const float b = bound_now();
     const float at = (b - GUMBEL_MAX) * temp;
@@ -350,93 +457,90 @@ __global__ __launch_bounds__(THREADS, TY == LOGITS_F32 ? 4 : 8) void sample_part
       queued -= n;
       if (lane < n) {
         const Pending p = queue[queued + lane];
-        visit(p.col, p.x);
+        const float u = uniform(p.col);
+        if (!loses(p.x, u)) visit(p.col, p.x, u);
       }
     }
     wave_lds_fence();
   };
-  if (!noisy) {  // the largest logit: tiles without one that reaches the bound are passed over
-    constexpr bool AHEAD = TY != LOGITS_F32 && THREADS == 1024;  // the next tile in flight (two of float32 would spill)
-    Chunk<TY> next[SAMPLE_IT];
-    auto advance = [&](int64_t base) {
-      if (AHEAD) {
-#pragma unroll
-        for (int it = 0; it < SAMPLE_IT; ++it) x[it] = next[it];
-      } else if (base < a.vocab) {
-        load(x, base);
-      }
-    };
-    for (int64_t base = first; base < a.vocab; base += hop, advance(base)) {
-      if (AHEAD && base + hop < a.vocab) load(next, base + hop);
-      if (base != first) {
-        const float b = bound_now();
-        bool any = false;
-#pragma unroll
-        for (int it = 0; it < SAMPLE_IT; ++it)
-#pragma unroll
-          for (int j = 0; j < 8; ++j) any |= !(x[it].at(j) < b);
-        if (__ballot(any) == 0) continue;
-      }
-      const int64_t col0 = base + 8 * (int)threadIdx.x;
-      const int32_t left = left_of(col0);
+  for (uint32_t g = first;;) {
+    const uint32_t col0 = col0_of(g);
+    bool take = true;
+    if (SEVERAL && g != first) {
+      lower();
+      bool nan;
+      const float m = tile_max<TY>(x, nan);
+      take = __ballot(!(m < low) || nan) != 0;
+    }
+    if (take) {
+      float top = x[0].at(0);
+      uint32_t at = 0;
 #pragma unroll
       for (int it = 0; it < SAMPLE_IT; ++it) {
-        x[it].forget();
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-          if (it * STEP + j < left) visit_next(bk, bi, x[it].at(j), (int32_t)col0 + it * STEP + j);
-      }
-      if (base + hop < a.vocab) raise(bk);
-    }
-    store_best<THREADS>(a, row, blockIdx.x, bk, bi);
-    return;
-  }
-  auto advance = [&](int64_t base) {
-    if (base < a.vocab) load(x, base);
-  };
-  for (int64_t base = first; base < a.vocab; base += hop, advance(base)) {
-    const int64_t col0 = base + 8 * (int)threadIdx.x;
-    const int32_t left = left_of(col0);
-    if (base != first) {
-      lower();
-      bool any = false;
-#pragma unroll
-      for (int it = 0; it < SAMPLE_IT; ++it)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) any |= !(x[it].at(j) < low);
-      if (__ballot(any) == 0) continue;
-    }
-#pragma unroll
-    for (int it = 0; it < SAMPLE_IT; ++it) x[it].forget();
-    float top = x[0].at(0);
-    int32_t at = 0;
-#pragma unroll
-    for (int it = 0; it < SAMPLE_IT; ++it)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const bool take = x[it].at(j) > top;
-        top = take ? x[it].at(j) : top;
-        at = take ? it * STEP + j : at;
-      }
-    raise(keyed(top, uniform((int32_t)col0 + at)));  // past the vocabulary top is -inf: no bound from it
-    if (base == first) __syncthreads();  // every wavefront's, before any logit is taken
-    lower();
-#pragma unroll
-    for (int it = 0; it < SAMPLE_IT; ++it) {
-      x[it].forget();
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const bool can = !(x[it].at(j) < low) && it * STEP + j < left;
-        const uint64_t mask = __ballot(can);
-        if (mask != 0) {
-          const int before =
-              __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
-          if (can) queue[queued + before] = Pending{(int32_t)col0 + it * STEP + j, x[it].at(j)};
-          queued += __popcll(mask);
+        for (int j = 0; j < 8; ++j) {
+          const bool more = x[it].at(j) > top;
+          top = more ? x[it].at(j) : top;
+          at = more ? it * STEP + j : at;
         }
-        if ((j & 3) == 3 && queued >= 64) drain(63);
+        x[it].forget();
+      }
+      raise(keyed(top, uniform(col0 + at)));  // around the row top is -inf: no bound from it
+      if (g == first) __syncthreads();        // every wavefront's, before any logit is taken
+      lower();
+      int likely = 0;  // of 512 logits
+#pragma unroll
+      for (int j = 0; j < 8; ++j) likely += __popcll(__ballot(!(x[0].at(j) < low)));
+      x[0].forget();
+      if (likely > SAMPLE_DIRECT) {  // most can win: each lane takes its own, without the queue
+#pragma unroll 1
+        for (uint32_t h = g; h < g + CHUNKS && h < chunks; h += THREADS) {
+          if (h + threadIdx.x < chunks) {
+            Chunk<TY> c = view.chunk(h + threadIdx.x);
+            if (view.edge(h, THREADS)) view.trim(c, h + threadIdx.x);
+#pragma unroll
+            for (int j = 0; j < 8; j += 4) {  // four at a time: their Philox rounds overlap
+              float u[4];
+              bool any = false;
+#pragma unroll
+              for (int k = 0; k < 4; ++k) {
+                u[k] = uniform(col0_of(h) + j + k);
+                any |= !loses(c.at(j + k), u[k]);
+              }
+              if (any) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                  if (!loses(c.at(j + k), u[k])) visit(col0_of(h) + j + k, c.at(j + k), u[k]);
+              }
+            }
+          }
+          if (SEVERAL || h + THREADS < chunks) {
+            raise(bk);
+            lower();
+          }
+        }
+      } else {
+#pragma unroll
+        for (int it = 0; it < SAMPLE_IT; ++it) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            const bool can = !(x[it].at(j) < low);
+            const uint64_t mask = __ballot(can);
+            if (mask != 0) {
+              const int before =
+                  __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
+              if (can) queue[queued + before] = Pending{col0 + it * STEP + j, x[it].at(j)};
+              queued += __popcll(mask);
+            }
+            if ((j & 3) == 3 && queued >= 64) drain(63);
+          }
+        }
       }
     }
+    g += hop;
+    if (!SEVERAL || g >= chunks) break;
+    load(x, g);
+    trim(x, g);
   }
   drain(0);
   store_best<THREADS>(a, row, blockIdx.x, bk, bi);
@@ -500,20 +604,41 @@ static size_t select_ws_offset(int64_t rows, int64_t n_tiles) {
 // step per workgroup. us, 256 x 151936, 256 / 1024 threads: T = 0.9 66 / 62, 1.2 79 / 86,
 // equal logits 94 / 107, all greedy 29 / 28 (every logit drawn for: 91, and 25 all greedy); 400 rows, T = 0.9 92 /
 // 70, 1.2 112 / 120, all greedy 40 / 33 (136, and 33).
-static int sample_threads(int64_t rows, int64_t vocab) {
-  return rows * ((vocab + sample_tile(1024) - 1) / sample_tile(1024)) < 1600 ? 256 : 1024;
-}
-static int64_t sample_parts(int64_t rows, int64_t vocab) {
-  const int threads = sample_threads(rows, vocab);
-  const int64_t steps = (vocab + sample_tile(threads) - 1) / sample_tile(threads);
-  if (threads == 256) return steps;
-  const int64_t fill = 512 / rows > steps / 8 ? 512 / rows : steps / 8;
-  const int64_t each = fill <= 1 ? steps : (steps + fill - 1) / fill;
-  return (steps + each - 1) / each;
-}
+// How the sampler takes a call: threads per workgroup and workgroups per row.
+struct SamplePlan {
+  int threads;
+  int64_t parts;
+};
+// Logits from which a call's workgroups carry their bound over several tiles. Below, one
+// 256-thread tile each spreads best; us, 256 threads / 512 threads over two tiles, 304 x
+// 151936: T = 0.6 45 / -, 400 x 151936 (above): T = 0.6 56 / 48, 1.2 112 / 111, half greedy
+// 63 / 67, equal 131 / 139; 640 x 151936 79 / 66, 170 / 160, 94 / 90, 201 / 212.
+constexpr int64_t SAMPLE_LARGE = 50 << 20;
+// Rows of at most 2048 columns: one wavefront each from here on, below 256 threads that draw
+// for every logit (sample_short). 8192 x 1000: T = 0.6 18 us, equal logits 34 (36 with 256
+// threads); 2048 x 2040, equal logits: 20 against 17.5.
+constexpr int64_t SAMPLE_NARROW_ROWS = 4096;
 
-static int64_t select_slots(int64_t rows, int64_t vocab, bool sample) {
-  return sample ? sample_parts(rows, vocab) : (vocab + SEL_TILE - 1) / SEL_TILE;
+// The columns that a row's chunks may cover: its logits and, where rows are not 16-byte
+// aligned, those before it in its first granule.
+static int64_t sample_span(int64_t vocab, bool vec) { return vec ? vocab : vocab + 7; }
+
+// Large calls on 2-byte logits: one 1024-thread workgroup per row, whose bound is the row's
+// own, where the rows fill the CUs evenly (the last round of rows at least 95 % full);
+// elsewhere the CUs with a row more would set the time (640 x 151936, equal logits: 251 us
+// against 212), and 512 threads take two tiles each. us, 1024 x 151936, 1024 threads / 512:
+// T = 0.6 76 / 98, 1.2 202 / 243, half greedy 138 / 129, equal 333 / 327. Float32 tiles leave
+// room for half the wavefronts there (equal logits 390 us against 321 with 256 threads).
+static SamplePlan sample_plan(int64_t rows, int64_t vocab, bool vec, bool half) {
+  const int64_t span = sample_span(vocab, vec);
+  auto tiles = [&](int threads) { return (span + sample_tile(threads) - 1) / sample_tile(threads); };
+  if (span <= sample_tile(64) && rows >= SAMPLE_NARROW_ROWS) return SamplePlan{64, 1};
+  if (!half || span <= sample_tile(512) || rows * vocab < SAMPLE_LARGE) return SamplePlan{256, tiles(256)};
+  DeviceInfo info;
+  const int64_t cus = device_info(&info) == FM_OK ? info.cus : 256;
+  const int64_t rounds = (rows + cus - 1) / cus;
+  if (span > 2 * sample_tile(1024) && 20 * rounds * cus <= 21 * rows) return SamplePlan{1024, 1};
+  return SamplePlan{512, (tiles(512) + 1) / 2};
 }
 
 static int run_select(const void *logits, int32_t dtype, int64_t rows, int64_t vocab, int64_t row_stride,
@@ -529,16 +654,18 @@ static int run_select(const void *logits, int32_t dtype, int64_t rows, int64_t v
   FM_REQUIRE(row_stride >= vocab, "row stride %lld below the vocabulary %lld", (long long)row_stride,
              (long long)vocab);
   const bool sample = temps != nullptr;
-  const int64_t n_tiles = select_slots(rows, vocab, sample);
+  const int es = dtype == LOGITS_F32 ? 4 : 2;
+  const bool vec = (uintptr_t)logits % 16 == 0 && row_stride * es % 16 == 0;
+  const SamplePlan plan = sample_plan(rows, vocab, vec, es == 2);
+  const int64_t n_tiles = sample ? plan.parts : (vocab + SEL_TILE - 1) / SEL_TILE;
   const size_t need = select_ws_offset(rows, n_tiles) + (size_t)(rows * n_tiles) * sizeof(int32_t);
   if (ws_bytes < need) return fail(FM_ERR_WORKSPACE, "workspace of %zu bytes, %zu needed", ws_bytes, need);
-  const int es = dtype == LOGITS_F32 ? 4 : 2;
   SelectArgs a{};
   a.logits = (const char *)logits;
   a.row_bytes = row_stride * es;
   a.vocab = vocab;
   a.n_tiles = (int32_t)n_tiles;
-  a.vec = ((uintptr_t)logits % 16 == 0 && a.row_bytes % 16 == 0) ? 1 : 0;
+  a.vec = vec;
   a.temps = temps;
   a.greedy = greedy;
   a.seed = seed;
@@ -546,14 +673,20 @@ static int run_select(const void *logits, int32_t dtype, int64_t rows, int64_t v
   a.index = (int32_t *)((char *)ws + select_ws_offset(rows, n_tiles));
   hipStream_t s = (hipStream_t)stream;
   const dim3 grid((unsigned)n_tiles, (unsigned)rows);
-#define FM_SEL(TY)                                                                          \
-  do {                                                                                      \
-    if (sample && sample_threads(rows, vocab) == 1024)                                      \
-      hipLaunchKernelGGL((sample_parts_kernel<TY, 1024>), grid, dim3(1024), 0, s, a);         \
-    else if (sample)                                                                        \
-      hipLaunchKernelGGL((sample_parts_kernel<TY, 256>), grid, dim3(256), 0, s, a);           \
-    else                                                                                    \
-      hipLaunchKernelGGL((select_tiles_kernel<TY>), grid, dim3(SEL_THREADS), 0, s, a);        \
+#define FM_SAMPLE(TY, THREADS, SEVERAL) \
+  hipLaunchKernelGGL((sample_parts_kernel<TY, THREADS, SEVERAL>), grid, dim3(THREADS), 0, s, a)
+#define FM_SEL(TY)                                                                     \
+  do {                                                                                 \
+    if (!sample)                                                                       \
+      hipLaunchKernelGGL((select_tiles_kernel<TY>), grid, dim3(SEL_THREADS), 0, s, a); \
+    else if (plan.threads == 64)                                                       \
+      FM_SAMPLE(TY, 64, false);                                                        \
+    else if (TY == LOGITS_F32 || plan.threads == 256)                                  \
+      FM_SAMPLE(TY, 256, false);                                                       \
+    else if (plan.threads == 512)                                                      \
+      FM_SAMPLE(TY == LOGITS_F32 ? LOGITS_BF16 : TY, 512, true);                       \
+    else                                                                               \
+      FM_SAMPLE(TY == LOGITS_F32 ? LOGITS_BF16 : TY, 1024, true);                      \
   } while (0)
   if (dtype == LOGITS_BF16)
     FM_SEL(LOGITS_BF16);
@@ -562,6 +695,7 @@ static int run_select(const void *logits, int32_t dtype, int64_t rows, int64_t v
   else
     FM_SEL(LOGITS_F32);
 #undef FM_SEL
+#undef FM_SAMPLE
   FM_CHECK_HIP(hipGetLastError());
   hipLaunchKernelGGL(select_rows_kernel, dim3((unsigned)rows), dim3(64), 0, s, a.best, a.index, a.n_tiles, out);
   FM_CHECK_HIP(hipGetLastError());
@@ -574,7 +708,7 @@ using namespace fm;
 
 extern "C" size_t fm_select_workspace_bytes(int64_t rows, int64_t vocab) {
   if (rows <= 0 || vocab <= 0) return 0;
-  const int64_t n_tiles = (vocab + sample_tile(256) - 1) / sample_tile(256);  // the finest tiling: enough for both
+  const int64_t n_tiles = (sample_span(vocab, false) + sample_tile(256) - 1) / sample_tile(256);  // the finest tiling: enough for both
   return select_ws_offset(rows, n_tiles) + (size_t)(rows * n_tiles) * sizeof(int32_t);
 }
 

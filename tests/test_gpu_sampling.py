@@ -128,6 +128,91 @@ def test_sample_rows_special_rows(dev):
     assert int(got[5]) == int(x[5].float().argmax())
 
 
+# Rows, vocabulary and row stride of every way a call is taken, well inside each: one wavefront
+# per row, 256 threads over a short row and over single tiles, 512 threads over two tiles, and
+# 1024 over a whole row (for 2-byte logits; float32 takes 256 throughout); the last two pairs
+# once with 16-byte-aligned rows and once without.
+_PLANS = [(5000, 1003, 1003), (4096, 2041, 2048), (70, 2041, 2041), (60, 8200, 8200), (30, 50001, 50008),
+          (800, 66000, 66000), (700, 98309, 98309), (1024, 65544, 65544), (1024, 98309, 98309)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("rows,vocab,stride", _PLANS)
+def test_sample_rows_tiles_and_parts(dev, dtype, rows, vocab, stride):
+    """Greedy and sampled rows in one call whose winners, ties, NaN, infinities and -inf
+    stretches lie in the first, a later and the last tile: greedy rows exactly, sampled rows
+    of every kind the token that the noise of every logit selects."""
+    print(f"sample rows={rows} vocab={vocab} stride={stride} {dtype}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(rows + vocab)
+    x = torch.randn(rows, stride, generator=g, device=dev).to(dtype)
+    temps = 0.6 + 0.6 * torch.rand(rows, generator=g, device=dev)
+    late, mid, last = vocab - vocab // 8, vocab // 2 + 3, vocab - 1
+    kinds = 10
+    for r in [k + part for k in range(kinds) for part in (0, rows // 3 // kinds * kinds, rows // 2 // kinds * kinds)]:
+        k = r % kinds
+        if k == 1:  # the largest far on, twice: the first wins if greedy
+            x[r, late], x[r, last] = 20.0, 20.0
+        elif k == 2:
+            x[r, 1], x[r, mid] = 20.0, 20.0
+        elif k == 3:
+            x[r] = 0.5  # all equal
+        elif k == 4:
+            x[r] = -torch.inf
+        elif k == 5:
+            x[r, :late] = -torch.inf  # nothing before the last part
+        elif k == 6:
+            x[r, mid:] = -torch.inf
+        elif k == 7:
+            x[r, late], x[r, last] = torch.nan, torch.nan
+        elif k == 8:
+            x[r, mid] = torch.inf
+        elif k == 9:
+            temps[r] = 40.0
+    pick = torch.arange(rows, device=dev)
+    greedy = (pick // kinds) % 2 == 1
+    x[:, vocab:] = 30000.0  # what lies between the rows is no logit
+    seed = 0x7_1234_5678
+    x = x[:, :vocab]
+    got = ops.sample_rows(x, temps, greedy, torch.tensor(seed, device=dev)).cpu()
+    assert int(got.min()) >= 0 and int(got.max()) < vocab
+    want = torch.from_numpy(S.argmax_first(x[greedy].float().cpu().numpy()))
+    assert torch.equal(got[greedy.cpu()], want)
+    for r in [r for r in list(range(kinds)) + list(range(rows - 20, rows)) if not greedy[r]]:
+        row = x[r:r + 1].cpu()
+        keys = _all_keys(row, temps[r:r + 1].cpu(), seed, row0=r)[0]
+        best, won = S.argmax_first(keys[None])[0], int(got[r])
+        if np.isnan(keys).any() or not np.isfinite(keys[best]):
+            assert won == best, (r, won, best)
+        else:  # as in test_sample_rows_skips_only_losers
+            assert keys[won] >= keys[best] - 1e-5 - 4 * 2.0 ** -23 * abs(keys[best]), (r, won, best)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_sample_rows_any_alignment(dev, dtype):
+    """Rows that begin at every place of a 16-byte granule and end at every place of one,
+    between values that would win: sampled rows exactly the oracle's (its clear winners),
+    greedy rows its argmax, rows of -inf the first index."""
+    g = gen(11)
+    for vocab in (1, 2, 7, 8, 9, 63, 2040, 2041, 2047, 2048, 2049, 8191, 8192, 8193, 16385):
+        for offset in range(8):
+            rows, stride = 4, vocab + 3
+            buf = torch.full((rows * stride + 16,), 30000.0).to(dtype)
+            view = buf[offset:offset + rows * stride].view(rows, stride)
+            logits = torch.randn(rows, vocab, generator=g).to(dtype)
+            logits[3] = -torch.inf
+            view[:, :vocab] = logits
+            d = buf.to(dev)
+            x = torch.as_strided(d, (rows, vocab), (stride, 1), offset)
+            temps = 0.3 + torch.rand(rows, generator=g)
+            greedy = torch.tensor([False, True, False, offset % 2 == 0])
+            got = ops.sample_rows(x, temps.to(dev), greedy.to(dev), torch.tensor(99, device=dev)).cpu()
+            keys = S.sample_keys(logits.float().numpy(), temps.numpy(), greedy.numpy(), 99)
+            want = S.argmax_first(keys)
+            for r in range(rows):
+                clear = vocab == 1 or r == 3 or np.diff(np.sort(keys[r])[-2:])[0] > 1e-4 or greedy[r]
+                assert not clear or int(got[r]) == want[r], (vocab, offset, r)
+
+
 def test_sample_rows_offsets_wrap_past_int32(dev):
     """row * V + col passes 2^31 for the last rows: int32 arithmetic, as the reference's."""
     rows, vocab = 300, 7_300_000
