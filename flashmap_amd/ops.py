@@ -1222,10 +1222,16 @@ def _linear_streams(rows: int, n: int, k: int) -> bool:
     return (rows <= 16 and k <= 4096) or (rows <= LINEAR_ROWS and k <= 2048 and n <= 4096)
 
 
+def _followed() -> bool:
+    """Whether a compiler or tracer follows the call (torch.compile, torch.export, jit.trace;
+    a symbolic tracer's values show by their type)."""
+    return torch.compiler.is_compiling() or torch.jit.is_tracing()
+
+
 def _eager_here(*tensors: torch.Tensor | None) -> bool:
     """Whether a plain kernel launch is all that a call on these tensors asks for: CUDA
     tensors, no gradient (backward or forward mode), and nothing that watches or rewrites
-    torch's calls (autocast, subclasses and modes, functorch's transforms, tracers)."""
+    torch's calls (autocast, subclasses and modes, functorch's transforms)."""
     given = [t for t in tensors if t is not None]
     return (
         all(t.is_cuda and type(t) in (torch.Tensor, torch.nn.Parameter) for t in given)
@@ -1235,23 +1241,23 @@ def _eager_here(*tensors: torch.Tensor | None) -> bool:
         and torch._C._len_torch_dispatch_stack() == 0
         and torch._C._functorch.peek_interpreter_stack() is None
         and torch.autograd.forward_ad._current_level < 0
-        and not torch.jit.is_tracing()
-        and not torch.compiler.is_compiling()
     )
 
 
-def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
-    """``F.linear``. Few bf16 rows, which only stream the weights (``_linear_streams``),
-    run the framework's kernel (fm_linear_rows); the rest, and calls that ask for more than
-    a launch (``_eager_here``), torch's."""
-    k = weight.shape[-1]
-    if not x.is_cuda or x.numel() > LINEAR_ROWS * k:  # most calls: no further looks
-        return torch.nn.functional.linear(x, weight, bias)
+def linear_rows(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor | None:
+    """``F.linear`` of few bf16 rows, which only stream the weights (``_linear_streams``), by
+    fm_linear_rows; None for every other call and for those that ask for more than a launch
+    (``_eager_here``). What a compiler or tracer follows is decided first, before anything
+    of ``x`` is looked at: their graphs hold torch's Linear alone."""
+    if _followed() or type(x) is not torch.Tensor or not x.is_cuda or weight.dim() != 2:
+        return None
+    n, k = weight.shape
+    if x.numel() > LINEAR_ROWS * k:  # most calls: no further looks
+        return None
     rows = x.numel() // k if k else 0
-    if (
+    if not (
         rows > 0
-        and weight.dim() == 2
-        and _linear_streams(rows, weight.shape[0], k)
+        and _linear_streams(rows, n, k)
         and x.shape[-1] == k
         and x.dtype == weight.dtype == torch.bfloat16
         and (bias is None or (bias.dtype == torch.bfloat16 and bias.is_contiguous() and bias.shape == weight.shape[:1]))
@@ -1265,12 +1271,17 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
         and x.data_ptr() % 16 == 0
         and weight.data_ptr() % 16 == 0
     ):
-        n = weight.shape[0]
-        out = torch.empty(*x.shape[:-1], n, dtype=torch.bfloat16, device=x.device)
-        call("fm_linear_rows", x.data_ptr(), k, weight.data_ptr(), weight.stride(0), _ptr(bias), out.data_ptr(), n,
-             rows, n, k, _stream(x))
-        return out
-    return torch.nn.functional.linear(x, weight, bias)
+        return None
+    out = torch.empty(*x.shape[:-1], n, dtype=torch.bfloat16, device=x.device)
+    call("fm_linear_rows", x.data_ptr(), k, weight.data_ptr(), weight.stride(0), _ptr(bias), out.data_ptr(), n,
+         rows, n, k, _stream(x))
+    return out
+
+
+def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
+    """``F.linear``, by the framework's kernel where :func:`linear_rows` takes the call."""
+    out = linear_rows(x, weight, bias)
+    return torch.nn.functional.linear(x, weight, bias) if out is None else out
 
 
 def noise_rows(z: torch.Tensor, eigvals: torch.Tensor, eps: float, gain: float,

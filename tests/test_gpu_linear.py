@@ -8,9 +8,17 @@ import torch
 import torch.nn.functional as F
 
 from _inputs import gen
-from flashmap_amd import ops
+from flashmap_amd import drafter, ops
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def launches(monkeypatch):
+    """The native calls made, by name."""
+    made, call = [], ops.call
+    monkeypatch.setattr(ops, "call", lambda name, *args: (made.append(name), call(name, *args))[1])
+    return made
 
 
 def _bound(x, w, bias, ref):
@@ -23,7 +31,7 @@ def _bound(x, w, bias, ref):
 @pytest.mark.parametrize("rows,n,k", [(1, 1, 32), (16, 100, 64), (15, 17, 1376), (16, 4097, 2048), (16, 8192, 2048),
                                       (16, 2048, 4096), (17, 2048, 2048), (32, 4096, 1056), (31, 33, 544)])
 @pytest.mark.parametrize("with_bias", [False, True])
-def test_linear_rows(dev, rows, n, k, with_bias):
+def test_linear_rows(dev, launches, rows, n, k, with_bias):
     print(f"linear rows={rows} n={n} k={k}", flush=True)
     g = gen(rows + n + k)
     x = torch.randn(rows, k, generator=g).bfloat16()
@@ -34,17 +42,22 @@ def test_linear_rows(dev, rows, n, k, with_bias):
         wd = w.to(dev) if w.is_contiguous() else wide.to(dev)[:, :k]
         got = ops.linear(x.to(dev), wd, None if bias is None else bias.to(dev)).cpu()
         ref = x.double() @ w.double().T + (0 if bias is None else bias.double())
+        assert launches == ["fm_linear_rows"], "the kernel and not the library"
+        launches.clear()
         assert got.shape == (rows, n) and got.dtype == torch.bfloat16
         assert ((got.double() - ref).abs() <= _bound(x, w, bias, ref)).all()
 
 
-def test_leading_dimensions_and_fallbacks(dev):
+def test_leading_dimensions_and_fallbacks(dev, launches):
     g = gen(3)
     x = torch.randn(2, 5, 64, generator=g).bfloat16().to(dev)
     w = torch.randn(48, 64, generator=g).bfloat16().to(dev)
     got = ops.linear(x, w)
     assert got.shape == (2, 5, 48)
     assert torch.equal(got.view(10, 48), ops.linear(x.view(10, 64), w))
+    assert ops.linear(x[0, 0], w).shape == (48,)
+    assert launches == ["fm_linear_rows"] * 3
+    launches.clear()
     # gradients, other types and strided rows go to torch, with its results
     wp = w.clone().requires_grad_(True)
     ops.linear(x, wp).float().sum().backward()
@@ -54,10 +67,45 @@ def test_leading_dimensions_and_fallbacks(dev):
     assert torch.equal(ops.linear(x.float(), w.float()), F.linear(x.float(), w.float()))
     strided = torch.randn(10, 128, generator=g).bfloat16().to(dev)[:, ::2]
     assert torch.equal(ops.linear(strided, w), F.linear(strided, w))
+    off = torch.randn(10 * 64 + 1, generator=g).bfloat16().to(dev)[1:].view(10, 64)  # not 16-byte aligned
+    assert torch.equal(ops.linear(off, w), F.linear(off, w))
     with torch.autocast("cuda", dtype=torch.float16):
         assert ops.linear(x, w).dtype == torch.float16
     with torch.no_grad():
         mapped = torch.func.vmap(lambda row: ops.linear(row, w))(x.view(10, 64))
     assert torch.equal(mapped, torch.func.vmap(lambda row: F.linear(row, w))(x.view(10, 64)))
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(x, torch.ones_like(x))
+        tangent = torch.autograd.forward_ad.unpack_dual(ops.linear(dual, w)).tangent
+    assert torch.equal(tangent, F.linear(torch.ones_like(x), w))
     with pytest.raises(RuntimeError):
         ops.linear(x[..., :32], w)
+    with pytest.raises(RuntimeError):
+        ops.linear(x[0, 0, 0], w)
+    assert launches == []
+
+
+def test_modules_take_the_kernel_and_keep_their_hooks(dev, launches):
+    torch.manual_seed(5)
+    cfg = drafter.drafter_config(hidden_size=64, num_attention_heads=2, intermediate_size=96)
+    mlp = drafter.FlashMapMLP(cfg).bfloat16().to(dev)
+    x = torch.randn(16, 64, device=dev).bfloat16()
+    with torch.no_grad():
+        want = F.linear(F.gelu(F.linear(x, mlp.fc1.weight, mlp.fc1.bias)), mlp.fc2.weight, mlp.fc2.bias)
+        got = mlp(x)
+        assert launches == ["fm_linear_rows"] * 2
+        # two bf16 roundings (2^-8 each) between sums in another order
+        assert float((got.double() - want.double()).norm() / want.double().norm()) < 2 ** -7
+        launches.clear()
+        torch._dynamo.reset()
+        assert torch.equal(torch.compile(mlp, fullgraph=True, backend="eager")(x), want)
+        assert torch.equal(torch.jit.trace(mlp, x, check_trace=False)(x), want)
+        assert launches == []
+        seen = []
+        mlp.fc1.register_forward_hook(lambda m, args, out: seen.append(out))
+        hooked = mlp(x)
+        assert len(seen) == 1 and launches == ["fm_linear_rows"]  # fc2's
+        assert torch.equal(hooked, ops.linear(F.gelu(seen[0]), mlp.fc2.weight, mlp.fc2.bias))
+    launches.clear()
+    mlp(x).float().sum().backward()
+    assert mlp.fc1.weight.grad is not None and launches == []
