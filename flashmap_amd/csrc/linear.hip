@@ -11,8 +11,8 @@
 //              as loaded (16 bytes per lane: row lane % 16, k 8 * (lane / 16))
 //   LDS:       (wavefront, row block, lane) fp32x4, summed by one wavefront per row block
 // bias is added in fp32 before the one rounding to bf16.
-// Measured (weights from HBM, 16 rows, this kernel and the library's): 2048 x 2048 7.0 us
-// (1.2 TB/s) and 10.7, 8192 x 2048 12.3 (2.7 TB/s) and 12.7; one row reads x from one line
+// Measured (weights from HBM, 16 rows, this kernel and the library's): 2048 x 2048 6.7 us
+// (1.25 TB/s) and 11.1, 8192 x 2048 12.6 (2.7 TB/s) and 14.5; one row reads x from one line
 // and takes 5.5 and 9.6 us: past the launch it is the reads of x, as many bytes as the
 // weights and all of them from L2, that a second row block doubles.
 #include <stdint.h>

@@ -163,7 +163,9 @@ def _project(module: nn.Module, x: torch.Tensor) -> torch.Tensor:
     """``module(x)`` for an ``nn.Linear``, few rows by the framework's kernel
     (:func:`ops.linear_rows`). Under a compiler or tracer, and for whatever else was put in
     the module's place or around it, the module's own call."""
-    if ops._followed() or type(x) is not torch.Tensor or not x.is_cuda or not _bare(module):
+    if ops._followed() or type(x) is not torch.Tensor or not x.is_cuda:
+        return module(x)
+    if x.dim() == 0 or x.numel() > ops.LINEAR_ROWS * x.shape[-1] or not _bare(module):
         return module(x)
     y = ops.linear_rows(x, module.weight, module.bias)
     return module(x) if y is None else y

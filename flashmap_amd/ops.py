@@ -1213,13 +1213,17 @@ def _linear_streams(rows: int, n: int, k: int) -> bool:
     """Whether fm_linear_rows is the faster one: sixteen rows of it read no more than the
     weights do, and past them (or long reductions, or the wide heads) the rows that every
     workgroup reads again cost more than the library's tiling. Measured, us, this kernel
-    and the library's, weights from HBM: 16 rows, n x k 2048 x 2048 7.0 / 10.7, 6144 x 2048
-    11.7 / 12.2, 8192 x 2048 12.3 / 12.7, 2048 x 4096 11.2 / 14.6, 2048 x 8192 19.7 / 12.9,
-    32000 x 4096 80 / 57; 32 rows, 2048 x 2048 9.5 / 10.9, 4096 x 2048 10.5 / 11.7, 6144 x
-    2048 16.5 / 12.3."""
-    if k % 32 or not 0 < n <= 8192:
+    and the library's, weights from HBM, n x k at 16 rows: 2048 x 256 3.2 / 3.8, 2048 x 2048
+    6.7 / 11.1, 6144 x 2048 11.8 / 12.9, 8192 x 2048 12.6 / 14.5, 64 x 4096 9.0 / 10.6, 2048 x
+    4096 10.8 / 14.8, 4096 x 4096 12.9 / 15.8; past the lines 6144 x 3072 17.0 / 13.4, 6144 x
+    4096 21.2 / 16.0, 8192 x 4096 23.2 / 17.5, 2048 x 8192 19.7 / 12.9, 32000 x 4096 80 / 57.
+    At 32 rows 64 x 2048 7.5 / 7.8, 2048 x 2048 9.2 / 11.3, 4096 x 2048 10.0 / 11.9; past them
+    6144 x 2048 16.5 / 12.3."""
+    if k % 32 or n <= 0 or rows > LINEAR_ROWS:
         return False
-    return (rows <= 16 and k <= 4096) or (rows <= LINEAR_ROWS and k <= 2048 and n <= 4096)
+    if rows > 16:
+        return n <= 4096 and k <= 2048
+    return (n <= 4096 and k <= 4096) or (n <= 8192 and k <= 2048)
 
 
 def _followed() -> bool:

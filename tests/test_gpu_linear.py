@@ -29,7 +29,7 @@ def _bound(x, w, bias, ref):
 
 
 @pytest.mark.parametrize("rows,n,k", [(1, 1, 32), (16, 100, 64), (15, 17, 1376), (16, 4097, 2048), (16, 8192, 2048),
-                                      (16, 2048, 4096), (17, 2048, 2048), (32, 4096, 1056), (31, 33, 544)])
+                                      (16, 2048, 4096), (16, 4096, 4096), (17, 2048, 2048), (32, 4096, 1056), (31, 33, 544)])
 @pytest.mark.parametrize("with_bias", [False, True])
 def test_linear_rows(dev, launches, rows, n, k, with_bias):
     print(f"linear rows={rows} n={n} k={k}", flush=True)
@@ -46,6 +46,20 @@ def test_linear_rows(dev, launches, rows, n, k, with_bias):
         launches.clear()
         assert got.shape == (rows, n) and got.dtype == torch.bfloat16
         assert ((got.double() - ref).abs() <= _bound(x, w, bias, ref)).all()
+
+
+def test_two_row_blocks_of_eight_wavefronts(dev):
+    """The C entry's widest form (32 rows, more than a tile of columns per CU), which the rule
+    above leaves to the library."""
+    rows, n, k = 32, 8200, 96
+    g = gen(4)
+    x, w = torch.randn(rows, k, generator=g).bfloat16(), torch.randn(n, k, generator=g).bfloat16()
+    assert not ops._linear_streams(rows, n, k)
+    xd, wd, out = x.to(dev), w.to(dev), torch.empty(rows, n, dtype=torch.bfloat16, device=dev)
+    ops.call("fm_linear_rows", xd.data_ptr(), k, wd.data_ptr(), k, None, out.data_ptr(), n, rows, n, k,
+             torch.cuda.current_stream().cuda_stream)
+    ref = x.double() @ w.double().T
+    assert ((out.cpu().double() - ref).abs() <= _bound(x, w, None, ref)).all()
 
 
 def test_leading_dimensions_and_fallbacks(dev, launches):

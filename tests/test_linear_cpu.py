@@ -27,6 +27,8 @@ def test_cpu_calls_are_torchs():
 
 @pytest.mark.parametrize("rows,n,k,takes", [(16, 2048, 2048, True), (16, 8192, 2048, True), (16, 2048, 4096, True),
                                             (16, 2048, 8192, False), (16, 32000, 2048, False),
+                                            (16, 4096, 4096, True), (16, 4097, 2080, False), (16, 6144, 3072, False),
+                                            (1, 8192, 4096, False), (32, 4096, 2048, True),
                                             (17, 4096, 2048, True), (17, 6144, 2048, False), (33, 64, 64, False),
                                             (4, 64, 48, False), (4, 0, 64, False)])
 def test_rule(rows, n, k, takes):
