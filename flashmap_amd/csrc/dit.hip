@@ -201,6 +201,15 @@ struct DivBy {
   }
 };
 
+// The exponent of a value: what the product scale * x leaves of the row's max m (a rounded
+// product itself) in one rounding, or x - m. The same in the sum and in the outputs, which
+// therefore add up to 1 at any scale: at products of 4e6 the max is rounded by up to 0.25,
+// and an exponent that rounds the product first differs by a factor of up to 1.28.
+template <bool SCALED>
+__device__ __forceinline__ float below(float x, float scale, float m) {
+  return SCALED ? __builtin_fmaf(x, scale, -m) : x - m;
+}
+
 // m starts at the lowest finite value, so that no difference below is inf - inf unless a
 // value is +inf (the row is then NaN, as torch has it).
 struct RowStats {
@@ -219,15 +228,15 @@ struct RowStats {
   }
 };
 
-template <int N>
-__device__ __forceinline__ void add_values(RowStats &st, const float (&x)[N]) {
-  float mx = x[0];
+template <bool SCALED, int N>
+__device__ __forceinline__ void add_values(RowStats &st, const float (&x)[N], float scale) {
+  float mx = SCALED ? x[0] * scale : x[0];
 #pragma unroll
-  for (int q = 1; q < N; ++q) mx = fmaxf(mx, x[q]);
+  for (int q = 1; q < N; ++q) mx = fmaxf(mx, SCALED ? x[q] * scale : x[q]);
   st.raise(mx);
   float s = 0.f;
 #pragma unroll
-  for (int q = 0; q < N; ++q) s += exp_neg(x[q] - st.m);
+  for (int q = 0; q < N; ++q) s += exp_neg(below<SCALED>(x[q], scale, st.m));
   st.s += s;
 }
 
@@ -269,8 +278,9 @@ __device__ __forceinline__ void store_last(T *p, V v) {
 __device__ __forceinline__ float load1(const float *p) { return *p; }
 __device__ __forceinline__ float load1(const uint16_t *p) { return bf16_to_f32(*p); }
 
-// Adds scale * x over the 4-value chunks [from, end) of a row to this thread's statistics.
-template <typename T>
+// Adds scale * x (SCALED; else x) over the 4-value chunks [from, end) of a row to this
+// thread's statistics.
+template <bool SCALED, typename T>
 __device__ __forceinline__ void add_chunks(RowStats &st, const T *x, int64_t from, int64_t end, float scale) {
   int64_t c = from + threadIdx.x;
   for (; c + (STATE_CHUNKS - 1) * STATE_THREADS < end; c += STATE_CHUNKS * STATE_THREADS) {
@@ -279,22 +289,22 @@ __device__ __forceinline__ void add_chunks(RowStats &st, const T *x, int64_t fro
     for (int k = 0; k < STATE_CHUNKS; ++k) {
       const f32x4_t v = load4(x + 4 * (c + k * STATE_THREADS));
 #pragma unroll
-      for (int q = 0; q < 4; ++q) e[4 * k + q] = v[q] * scale;
+      for (int q = 0; q < 4; ++q) e[4 * k + q] = v[q];
     }
-    add_values(st, e);
+    add_values<SCALED>(st, e, scale);
   }
   for (; c < end; c += STATE_THREADS) {
     const f32x4_t v = load4(x + 4 * c);
-    const float e[4] = {v[0] * scale, v[1] * scale, v[2] * scale, v[3] * scale};
-    add_values(st, e);
+    const float e[4] = {v[0], v[1], v[2], v[3]};
+    add_values<SCALED>(st, e, scale);
   }
 }
 // ... over the values past a row's last whole chunk (vocab % 4 of them).
-template <typename T>
+template <bool SCALED, typename T>
 __device__ __forceinline__ void add_tail(RowStats &st, const T *x, int64_t vocab, float scale) {
   for (int64_t i = (vocab & ~3ll) + threadIdx.x; i < vocab; i += STATE_THREADS) {
-    const float e[1] = {load1(x + i) * scale};
-    add_values(st, e);
+    const float e[1] = {load1(x + i)};
+    add_values<SCALED>(st, e, scale);
   }
 }
 
@@ -335,15 +345,14 @@ __global__ __launch_bounds__(STATE_THREADS) void state_embed_rows_kernel(const f
 #pragma unroll
     for (int k = 0; k < STATE_HELD; ++k) {
       if (c + k * STATE_THREADS < part.end) {
-        const float e[4] = {held[k][0] * evidence, held[k][1] * evidence, held[k][2] * evidence,
-                            held[k][3] * evidence};
-        add_values(t, e);
+        const float e[4] = {held[k][0], held[k][1], held[k][2], held[k][3]};
+        add_values<true>(t, e, evidence);
       }
     }
     const int64_t next = part.first + STATE_HELD * STATE_THREADS;
-    add_chunks(t, x, 0, part.first, evidence);
-    add_chunks(t, x, next < part.end ? next : part.end, chunks, evidence);
-    add_tail(t, x, vocab, evidence);
+    add_chunks<true>(t, x, 0, part.first, evidence);
+    add_chunks<true>(t, x, next < part.end ? next : part.end, chunks, evidence);
+    add_tail<true>(t, x, vocab, evidence);
     t = block_stats(t);
   }
   const DivBy div(t.s);
@@ -351,7 +360,7 @@ __global__ __launch_bounds__(STATE_THREADS) void state_embed_rows_kernel(const f
     if constexpr (POST) {
       float p[4];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) p[q] = div(exp_neg(v[q] * evidence - t.m));
+      for (int q = 0; q < 4; ++q) p[q] = div(exp_neg(below<true>(v[q], evidence, t.m)));
       store_last<NT>(post + 4 * c, u32x2_t{pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3])});
     }
     store_last<NT>(raw + 4 * c, u32x2_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])});
@@ -366,7 +375,7 @@ __global__ __launch_bounds__(STATE_THREADS) void state_embed_rows_kernel(const f
   if (!part.last) return;
   for (int64_t i = 4 * chunks + threadIdx.x; i < vocab; i += STATE_THREADS) {
     if constexpr (POST)
-      post[i] = (uint16_t)(pack_bf16x2(div(exp_neg(x[i] * evidence - t.m)), 0.f) & 0xffffu);
+      post[i] = (uint16_t)(pack_bf16x2(div(exp_neg(below<true>(x[i], evidence, t.m))), 0.f) & 0xffffu);
     raw[i] = (uint16_t)(pack_bf16x2(x[i], 0.f) & 0xffffu);
   }
 }
@@ -383,12 +392,12 @@ __global__ __launch_bounds__(STATE_THREADS) void state_update_kernel(float *__re
   const int64_t chunks = vocab >> 2;
   const PartOf part = part_of(chunks);
   RowStats t = RowStats::none();
-  add_chunks(t, lg, 0, chunks, 1.f);
-  add_tail(t, lg, vocab, 1.f);
+  add_chunks<false>(t, lg, 0, chunks, 1.f);
+  add_tail<false>(t, lg, vocab, 1.f);
   t = block_stats(t);
   const DivBy div(t.s), scale(c_div);
   auto upd = [&](float s, float l) {
-    return scale.any(c_keep * s + c_new * div(exp_neg(l - t.m)));
+    return scale.any(__builtin_fmaf(c_keep, s, c_new * div(exp_neg(l - t.m))));
   };
 #pragma unroll 4
   for (int64_t c = part.first + threadIdx.x; c < part.end; c += STATE_THREADS) {

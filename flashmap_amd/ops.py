@@ -1324,8 +1324,9 @@ def _state_rows(state: torch.Tensor) -> None:
 def state_embed_rows(state: torch.Tensor, evidence: float, out: torch.Tensor | None = None,
                      posterior: bool = True) -> torch.Tensor:
     """``torch.cat([softmax(evidence * state), state]).to(bf16)`` for the several-jump
-    draft's state ``(rows, vocab)`` float32 (flashmap/vllm/model.py:944-956): one kernel
-    reading each row twice, ``(2 rows, vocab)`` bf16, the operand of the state
+    draft's state ``(rows, vocab)`` float32 (flashmap/vllm/model.py:944-956), the products
+    ``evidence * state`` unrounded (torch rounds them to float32, which at large evidence
+    changes the posterior): one kernel reading each row twice, ``(2 rows, vocab)`` bf16, the operand of the state
     embedding's GEMM. ``posterior=False``: the state rows alone ``(rows, vocab)`` (one
     read), for a jump whose posterior is uniform."""
     _check_cuda(state, out)
@@ -1347,7 +1348,9 @@ def state_embed_rows(state: torch.Tensor, evidence: float, out: torch.Tensor | N
 def state_update(state: torch.Tensor, logits: torch.Tensor, start: float, end: float) -> torch.Tensor:
     """The state update between two jumps, in place (flashmap/vllm/model.py:1031-1036):
     ``state = ((1 - end) state + (end - start) softmax(logits)) / (1 - start)`` with
-    ``logits (rows, vocab)`` bf16, in float32 with torch's rounding points."""
+    ``logits (rows, vocab)`` bf16, in float32: the softmax rounded as torch rounds it (the
+    exponentials, their sum in another order, the quotient), then the first product and the
+    sum in one rounding and the quotient by ``1 - start``, the scalars rounded from double."""
     _check_cuda(state, logits)
     _state_rows(state)
     rows, vocab = state.shape

@@ -70,6 +70,25 @@ def test_state_update(dev, rows, vocab, start, end):
     assert torch.allclose(out.cpu().double().sum(-1), torch.ones(rows, dtype=torch.float64), atol=1e-4)
 
 
+@pytest.mark.parametrize("evidence", [1e3, 1e5, 1e6, -1e3])
+def test_posterior_at_large_evidence(dev, evidence):
+    """Products of up to 5e6, whose float32 rounding is up to a quarter: the posterior is that
+    of the exact products all the same, and adds up to 1."""
+    rows, vocab = 70, 5003
+    g = gen(int(abs(evidence)))
+    state = torch.randn(rows, vocab, generator=g)
+    peak = 4.5 if evidence > 0 else -4.5
+    state[:, 17] = peak + 0.1 * torch.rand(rows, generator=g)
+    state[:, 4999] = state[:, 17] - torch.rand(rows, generator=g) * 2 / evidence  # within two of it
+    got = ops.state_embed_rows(_rows(state, dev), evidence).cpu()[:rows].double()
+    want = torch.softmax(state.double() * evidence, dim=-1)
+    # an exponent's one float32 rounding and the exponential's are below 1e-4 of the value at
+    # exponents of -100 and more; then bf16's half ulp, 2^-8 of the value at most
+    seen = want > 1e-40
+    assert float(((got - want).abs() / want)[seen].max()) <= 2.0 ** -8
+    assert float(got.max()) <= 1.0 and float((got.sum(-1) - 1).abs().max()) <= 2.0 ** -8
+
+
 def test_state_kernels_strided_rows(dev):
     """Rows inside a wider buffer (the draft step's padded state), and the state update
     against torch's float32 expression on the same device."""
