@@ -176,17 +176,30 @@ constexpr int STATE_HELD = 8;    // state_embed_rows: chunks per thread kept bet
 
 // exp(x) for x <= 0 (0 for -inf, NaN for NaN) to about an ulp: exp2 of the rounded x log2(e),
 // corrected by what that rounding left of x. r is NaN only for x = -inf (the result is 0
-// already) and NaN (the result is NaN): the max keeps it out of the product.
+// already) and NaN (the result is NaN): the max keeps it out of the product. Results below
+// 2^-126 are 0 (the hardware's exp2 has no subnormals): for the sums, whose largest term is 1.
 __device__ __forceinline__ float exp_neg(float x) {
+#pragma clang fp contract(off)  // r is taken from the rounded t
   const float t = x * 1.44269504f;
   const float p = __builtin_amdgcn_exp2f(t);
-  float r = __builtin_fmaf(-t, 0.693147182f, x);
-  r = __builtin_fmaf(-t, -1.90465421e-9f, r);
+  const float r = __builtin_fmaf(-t, -1.90465421e-9f, __builtin_fmaf(-t, 0.693147182f, x));
   return __builtin_fmaf(p, fmaxf(r, -0.001f), p);
 }
 
-// a / c by c's reciprocal and one residual step: the rounded quotient but for rare
-// last-bit ties.
+// 2^24 exp(x), for the outputs, whose divisor carries the same factor: exp2's results are
+// normal wherever exp(x) is at least a subnormal. The subtraction is exact (u has t's grid
+// where it is the smaller of the two, and is within a factor of two of 24 elsewhere).
+constexpr float EXP_SCALE = 0x1p24f;
+__device__ __forceinline__ float exp_scaled(float x) {
+  const float u = __builtin_fmaf(x, 1.44269504f, 24.f);
+  const float p = __builtin_amdgcn_exp2f(u);
+  const float t = u - 24.f;
+  const float r = __builtin_fmaf(-t, -1.90465421e-9f, __builtin_fmaf(-t, 0.693147182f, x));
+  return __builtin_fmaf(p, fmaxf(r, -0.001f), p);
+}
+
+// a / c by c's correctly rounded reciprocal and one residual step: the rounded quotient
+// (4 x 10^6 random numerators over each of six divisors from 26 to 2843: no difference).
 struct DivBy {
   float c, y;
   __device__ __forceinline__ explicit DivBy(float c_) : c(c_), y(__fdiv_rn(1.0f, c_)) {}
@@ -355,12 +368,12 @@ __global__ __launch_bounds__(STATE_THREADS) void state_embed_rows_kernel(const f
     add_tail<true>(t, x, vocab, evidence);
     t = block_stats(t);
   }
-  const DivBy div(t.s);
+  const DivBy div(t.s * EXP_SCALE);
   auto put = [&](int64_t c, f32x4_t v) {
     if constexpr (POST) {
       float p[4];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) p[q] = div(exp_neg(below<true>(v[q], evidence, t.m)));
+      for (int q = 0; q < 4; ++q) p[q] = div(exp_scaled(below<true>(v[q], evidence, t.m)));
       store_last<NT>(post + 4 * c, u32x2_t{pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3])});
     }
     store_last<NT>(raw + 4 * c, u32x2_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])});
@@ -375,7 +388,7 @@ __global__ __launch_bounds__(STATE_THREADS) void state_embed_rows_kernel(const f
   if (!part.last) return;
   for (int64_t i = 4 * chunks + threadIdx.x; i < vocab; i += STATE_THREADS) {
     if constexpr (POST)
-      post[i] = (uint16_t)(pack_bf16x2(div(exp_neg(below<true>(x[i], evidence, t.m))), 0.f) & 0xffffu);
+      post[i] = (uint16_t)(pack_bf16x2(div(exp_scaled(below<true>(x[i], evidence, t.m))), 0.f) & 0xffffu);
     raw[i] = (uint16_t)(pack_bf16x2(x[i], 0.f) & 0xffffu);
   }
 }
@@ -395,9 +408,9 @@ __global__ __launch_bounds__(STATE_THREADS) void state_update_kernel(float *__re
   add_chunks<false>(t, lg, 0, chunks, 1.f);
   add_tail<false>(t, lg, vocab, 1.f);
   t = block_stats(t);
-  const DivBy div(t.s), scale(c_div);
+  const DivBy div(t.s * EXP_SCALE), scale(c_div);
   auto upd = [&](float s, float l) {
-    return scale.any(__builtin_fmaf(c_keep, s, c_new * div(exp_neg(l - t.m))));
+    return scale.any(__builtin_fmaf(c_keep, s, c_new * div(exp_scaled(l - t.m))));
   };
 #pragma unroll 4
   for (int64_t c = part.first + threadIdx.x; c < part.end; c += STATE_THREADS) {

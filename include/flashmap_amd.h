@@ -455,10 +455,10 @@ int fm_noise_rows(const float *z, int64_t rows, int32_t hidden, int64_t z_stride
  * `_embed_state`): for state (rows, vocab) fp32 with a row stride and posterior nonzero,
  * out rows r < rows get bf16(softmax(evidence * state[r])) and rows rows + r get
  * bf16(state[r]) -- the operand of the one GEMM through the state vocabulary's embedding
- * (torch.cat([posterior, state]).to(bf16)), the products evidence * state unrounded; out is (2 rows, vocab) bf16 with a row
- * stride. With posterior zero (a jump starting at time 0, whose posterior is uniform),
- * out is (rows, vocab): the state rows only. Strides multiples of 4; state 16-byte
- * aligned, out 8-byte aligned.
+ * (torch.cat([posterior, state]).to(bf16)), the products evidence * state unrounded; out
+ * is (2 rows, vocab) bf16 with a row stride. With posterior zero (a jump starting at time
+ * 0, whose posterior is uniform), out is (rows, vocab): the state rows only. Strides
+ * multiples of 4; state 16-byte aligned, out 8-byte aligned.
  */
 int fm_state_embed_rows(const float *state, int64_t rows, int64_t vocab, int64_t state_stride,
                         float evidence, int32_t posterior, void *out, int64_t out_stride, void *stream);

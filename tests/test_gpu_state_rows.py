@@ -89,6 +89,25 @@ def test_posterior_at_large_evidence(dev, evidence):
     assert float(got.max()) <= 1.0 and float((got.sum(-1) - 1).abs().max()) <= 2.0 ** -8
 
 
+def test_subnormal_probabilities(dev):
+    """Exponents around -87.3 to -104, whose float32 exponentials are subnormal: the posterior
+    keeps what bf16 has of them (steps of 2^-133), the update what float32 has (2^-149)."""
+    vocab = 4099
+    x = torch.linspace(-104.0, -80.0, vocab).repeat(2, 1)
+    x[:, 7] = 0.0
+    got = ops.state_embed_rows(_rows(x, dev), 1.0).cpu()[:2].double()
+    want = torch.softmax(x.double(), dim=-1)
+    assert int(((want < 2.0 ** -126) & (want > 2.0 ** -133)).sum()) > 1000
+    # float32's own rounding of the quotient, then half of bf16's step or of its value's ulp
+    assert ((got - want).abs() <= 2.0 ** -149 + 2.0 ** -134 + 2.0 ** -8 * want).all()
+    logits = x.bfloat16()
+    d64 = torch.softmax(logits.double(), dim=-1)
+    state = _rows(torch.zeros(2, vocab), dev)
+    out = ops.state_update(state, _rows(logits, dev), 0.0, 0.5).cpu().double()
+    # two roundings at 2^-149, and 1e-6 of the value as in test_state_update
+    assert ((out - 0.5 * d64).abs() <= 2.0 ** -148 + 1e-6 * d64).all()
+
+
 def test_state_kernels_strided_rows(dev):
     """Rows inside a wider buffer (the draft step's padded state), and the state update
     against torch's float32 expression on the same device."""
@@ -140,8 +159,9 @@ def test_state_kernels_edges(dev, rows, vocab):
     before = state.double()
     post = torch.softmax((1.5 * state).double(), -1)
     both = ops.state_embed_rows(state, 1.5)
-    # float32 exponentials and sums to about 1e-6, then bf16: an ulp is 2^-8 of the value
-    assert torch.allclose(both[:rows].double(), post, rtol=2.0 ** -8, atol=1e-37, equal_nan=True)
+    # float32 exponentials and sums to about 1e-6, then bf16: an ulp is 2^-8 of the value, and
+    # 2^-133 below its normal range
+    assert torch.allclose(both[:rows].double(), post, rtol=2.0 ** -8, atol=2.0 ** -133, equal_nan=True)
     assert torch.equal(both[rows:].view(torch.int16), state.bfloat16().view(torch.int16))
     want = (0.4 * before + 0.3 * torch.softmax(logits.double(), -1)) / 0.7
     out = ops.state_update(state, logits, 0.3, 0.6).double()
