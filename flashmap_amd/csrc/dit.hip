@@ -158,7 +158,9 @@ static bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 // The several-jump draft's state over the vocabulary (flashmap/vllm/model.py:944-956,
 // 1031-1036): softmaxes over rows of up to ~10^5 values. A row goes to `parts` workgroups
 // (state_parts); each forms the whole row's statistics (max and sum of exponentials,
-// online per thread, merged over the workgroup) and writes its part of the outputs.
+// online per thread, merged over the workgroup) and writes its part of the outputs. The
+// statistics are taken in one order whatever the part: a row's values do not depend on how
+// many rows the call has.
 //
 // Bound: HBM. Few rows are in flight (at most two 1024-thread workgroups per CU), so that
 // the second read of a row comes from the caches: with 256-thread workgroups each of 1024
@@ -335,8 +337,9 @@ __device__ __forceinline__ PartOf part_of(int64_t chunks) {
 
 // POST: rows r < rows of out get bf16(softmax(evidence * state[r])) and rows rows + r
 // bf16(state[r]); otherwise out holds the state rows only (one read of the row). A
-// workgroup keeps the first STATE_HELD chunks per thread of its part in registers between
-// the two passes (32768 values); the rest is read again from the caches.
+// workgroup keeps the row's first STATE_HELD chunks per thread in registers between the two
+// passes (32768 values), for the part that begins there; the rest is read again from the
+// caches.
 template <bool POST, bool NT>
 __global__ __launch_bounds__(STATE_THREADS) void state_embed_rows_kernel(const float *__restrict__ state,
                                                                          int64_t vocab, int64_t ss, float evidence,
@@ -349,22 +352,21 @@ __global__ __launch_bounds__(STATE_THREADS) void state_embed_rows_kernel(const f
   const PartOf part = part_of(chunks);
   RowStats t{0.f, 1.f};
   f32x4_t held[STATE_HELD];
-  int64_t c = part.first + threadIdx.x;
   if constexpr (POST) {
     t = RowStats::none();
 #pragma unroll
-    for (int k = 0; k < STATE_HELD; ++k)
-      held[k] = c + k * STATE_THREADS < part.end ? load4(x + 4 * (c + k * STATE_THREADS)) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int k = 0; k < STATE_HELD; ++k) {
+      const int64_t c = threadIdx.x + k * STATE_THREADS;
+      held[k] = c < chunks ? load4(x + 4 * c) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
 #pragma unroll
     for (int k = 0; k < STATE_HELD; ++k) {
-      if (c + k * STATE_THREADS < part.end) {
+      if (threadIdx.x + k * STATE_THREADS < chunks) {
         const float e[4] = {held[k][0], held[k][1], held[k][2], held[k][3]};
         add_values<true>(t, e, evidence);
       }
     }
-    const int64_t next = part.first + STATE_HELD * STATE_THREADS;
-    add_chunks<true>(t, x, 0, part.first, evidence);
-    add_chunks<true>(t, x, next < part.end ? next : part.end, chunks, evidence);
+    add_chunks<true>(t, x, STATE_HELD * STATE_THREADS, chunks, evidence);
     add_tail<true>(t, x, vocab, evidence);
     t = block_stats(t);
   }
@@ -378,10 +380,13 @@ __global__ __launch_bounds__(STATE_THREADS) void state_embed_rows_kernel(const f
     }
     store_last<NT>(raw + 4 * c, u32x2_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])});
   };
+  int64_t c = part.first + threadIdx.x;
   if constexpr (POST) {
+    if (part.first == 0) {
 #pragma unroll
-    for (int k = 0; k < STATE_HELD; ++k, c += STATE_THREADS)
-      if (c < part.end) put(c, held[k]);
+      for (int k = 0; k < STATE_HELD; ++k, c += STATE_THREADS)
+        if (c < part.end) put(c, held[k]);
+    }
   }
 #pragma unroll 4
   for (; c < part.end; c += STATE_THREADS) put(c, load_last<NT>(x + 4 * c));

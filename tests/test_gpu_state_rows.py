@@ -108,6 +108,23 @@ def test_subnormal_probabilities(dev):
     assert ((out - 0.5 * d64).abs() <= 2.0 ** -148 + 1e-6 * d64).all()
 
 
+@pytest.mark.parametrize("vocab", [1003, 32770, 49157, 151936])
+def test_rows_do_not_depend_on_the_others(dev, vocab):
+    """A row's values bit for bit, whether the call has 1, 16, 64, 200 or 300 rows (eight to
+    one workgroups a row)."""
+    print(f"state rows alone and together vocab={vocab}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(vocab)
+    state = _rows(torch.randn(300, vocab, generator=g, device=dev), dev)
+    logits = _rows(2 * torch.randn(300, vocab, generator=g, device=dev, dtype=torch.bfloat16), dev)
+    whole = ops.state_embed_rows(state, 3.0)
+    moved = ops.state_update(_rows(state, dev), logits, 0.2, 0.7)
+    for rows in (1, 16, 64, 200):
+        part = ops.state_embed_rows(state[:rows], 3.0)
+        assert torch.equal(part[:rows], whole[:rows]), (rows, "posterior")
+        assert torch.equal(part[rows:], whole[300:300 + rows]), (rows, "state")
+        assert torch.equal(ops.state_update(_rows(state[:rows], dev), logits[:rows], 0.2, 0.7), moved[:rows]), rows
+
+
 def test_state_kernels_strided_rows(dev):
     """Rows inside a wider buffer (the draft step's padded state), and the state update
     against torch's float32 expression on the same device."""
