@@ -162,17 +162,15 @@ static bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 // statistics are taken in one order whatever the part: a row's values do not depend on how
 // many rows the call has.
 //
-// Bound: HBM. Few rows are in flight (at most two 1024-thread workgroups per CU), so that
-// the second read of a row comes from the caches: with 256-thread workgroups each of 1024
-// rows was resident at once, 311 to 622 MB between the two reads. The arithmetic stays
-// below the stream: exponentials are exp_neg (9 issue slots against 18 for expf), the
-// divisions by a row's (or the call's) one divisor take its reciprocal once and three
-// operations per element (DivBy; 14 for an IEEE division). Measured, 1024 x 151936 (1.56
-// and 1.24 GB): update 422 -> 344 us with this arithmetic and these workgroups, 284 us with
-// the non-temporal second pass; embedding 400 -> 356 -> 284 us, 260 us with a quarter of the
-// row held (16 chunks held spill: 347 us). 512 threads per row: 312 and 266 us. In parts,
-// 64 rows: update 161 -> 42 us, embedding 155 -> 47 us; 16 rows: 123 -> 22, 111 -> 22 us.
-constexpr int STATE_THREADS = 1024;
+// Bound: HBM for a full batch over a whole vocabulary. Few rows are in flight there (one
+// 1024-thread workgroup per CU, or two), so that the second read of a row comes from the
+// caches: with 256-thread workgroups each of 1024 rows was resident at once, 311 to 622 MB
+// between the two reads. The arithmetic stays below the stream: exponentials are exp_neg (9
+// issue slots against 18 for expf), the divisions by a row's (or the call's) one divisor take
+// its reciprocal once and three operations per element (DivBy; 14 for an IEEE division), the
+// products' maximum one product. Measured, 1024 x 151936 (1.56 and 1.24 GB) with 256 threads,
+// expf and IEEE divisions / now: update 422 / 281 us, embedding 388 / 260 us (16 chunks held
+// spill: 347 us). In parts, 64 rows: update 162 / 42 us, embedding 153 / 38 us.
 constexpr int STATE_CHUNKS = 4;  // 4-value chunks in flight per thread
 constexpr int STATE_HELD = 8;    // state_embed_rows: chunks per thread kept between the passes
 
@@ -245,10 +243,17 @@ struct RowStats {
 
 template <bool SCALED, int N>
 __device__ __forceinline__ void add_values(RowStats &st, const float (&x)[N], float scale) {
-  float mx = SCALED ? x[0] * scale : x[0];
+  // The largest rounded product is the rounded product of the largest value (the smallest
+  // for a negative scale).
+  float mx = x[0];
+  if (SCALED && scale < 0.f) {
 #pragma unroll
-  for (int q = 1; q < N; ++q) mx = fmaxf(mx, SCALED ? x[q] * scale : x[q]);
-  st.raise(mx);
+    for (int q = 1; q < N; ++q) mx = fminf(mx, x[q]);
+  } else {
+#pragma unroll
+    for (int q = 1; q < N; ++q) mx = fmaxf(mx, x[q]);
+  }
+  st.raise(SCALED ? mx * scale : mx);
   float s = 0.f;
 #pragma unroll
   for (int q = 0; q < N; ++q) s += exp_neg(below<SCALED>(x[q], scale, st.m));
@@ -256,8 +261,9 @@ __device__ __forceinline__ void add_values(RowStats &st, const float (&x)[N], fl
 }
 
 // The workgroup's statistics from each thread's.
+template <int THREADS>
 __device__ __forceinline__ RowStats block_stats(RowStats st) {
-  __shared__ RowStats part[STATE_THREADS / 64];
+  __shared__ RowStats part[THREADS / 64];
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) {
     st.merge(RowStats{__shfl_xor(st.m, o, 64), __shfl_xor(st.s, o, 64)});
@@ -266,7 +272,7 @@ __device__ __forceinline__ RowStats block_stats(RowStats st) {
   __syncthreads();
   RowStats r = part[0];
 #pragma unroll
-  for (int w = 1; w < STATE_THREADS / 64; ++w) r.merge(part[w]);
+  for (int w = 1; w < THREADS / 64; ++w) r.merge(part[w]);
   return r;
 }
 
@@ -295,29 +301,29 @@ __device__ __forceinline__ float load1(const uint16_t *p) { return bf16_to_f32(*
 
 // Adds scale * x (SCALED; else x) over the 4-value chunks [from, end) of a row to this
 // thread's statistics.
-template <bool SCALED, typename T>
+template <int THREADS, bool SCALED, typename T>
 __device__ __forceinline__ void add_chunks(RowStats &st, const T *x, int64_t from, int64_t end, float scale) {
   int64_t c = from + threadIdx.x;
-  for (; c + (STATE_CHUNKS - 1) * STATE_THREADS < end; c += STATE_CHUNKS * STATE_THREADS) {
+  for (; c + (STATE_CHUNKS - 1) * THREADS < end; c += STATE_CHUNKS * THREADS) {
     float e[4 * STATE_CHUNKS];
 #pragma unroll
     for (int k = 0; k < STATE_CHUNKS; ++k) {
-      const f32x4_t v = load4(x + 4 * (c + k * STATE_THREADS));
+      const f32x4_t v = load4(x + 4 * (c + k * THREADS));
 #pragma unroll
       for (int q = 0; q < 4; ++q) e[4 * k + q] = v[q];
     }
     add_values<SCALED>(st, e, scale);
   }
-  for (; c < end; c += STATE_THREADS) {
+  for (; c < end; c += THREADS) {
     const f32x4_t v = load4(x + 4 * c);
     const float e[4] = {v[0], v[1], v[2], v[3]};
     add_values<SCALED>(st, e, scale);
   }
 }
 // ... over the values past a row's last whole chunk (vocab % 4 of them).
-template <bool SCALED, typename T>
+template <int THREADS, bool SCALED, typename T>
 __device__ __forceinline__ void add_tail(RowStats &st, const T *x, int64_t vocab, float scale) {
-  for (int64_t i = (vocab & ~3ll) + threadIdx.x; i < vocab; i += STATE_THREADS) {
+  for (int64_t i = (vocab & ~3ll) + threadIdx.x; i < vocab; i += THREADS) {
     const float e[1] = {load1(x + i)};
     add_values<SCALED>(st, e, scale);
   }
@@ -338,10 +344,10 @@ __device__ __forceinline__ PartOf part_of(int64_t chunks) {
 // POST: rows r < rows of out get bf16(softmax(evidence * state[r])) and rows rows + r
 // bf16(state[r]); otherwise out holds the state rows only (one read of the row). A
 // workgroup keeps the row's first STATE_HELD chunks per thread in registers between the two
-// passes (32768 values), for the part that begins there; the rest is read again from the
-// caches.
-template <bool POST, bool NT>
-__global__ __launch_bounds__(STATE_THREADS) void state_embed_rows_kernel(const float *__restrict__ state,
+// passes (32768 values of 1024 threads), for the part that begins there; the rest is read
+// again from the caches.
+template <bool POST, bool NT, int THREADS>
+__global__ __launch_bounds__(THREADS) void state_embed_rows_kernel(const float *__restrict__ state,
                                                                          int64_t vocab, int64_t ss, float evidence,
                                                                          uint16_t *__restrict__ out, int64_t os,
                                                                          int64_t rows) {
@@ -356,19 +362,29 @@ __global__ __launch_bounds__(STATE_THREADS) void state_embed_rows_kernel(const f
     t = RowStats::none();
 #pragma unroll
     for (int k = 0; k < STATE_HELD; ++k) {
-      const int64_t c = threadIdx.x + k * STATE_THREADS;
+      const int64_t c = threadIdx.x + k * THREADS;
       held[k] = c < chunks ? load4(x + 4 * c) : f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
 #pragma unroll
-    for (int k = 0; k < STATE_HELD; ++k) {
-      if (threadIdx.x + k * STATE_THREADS < chunks) {
-        const float e[4] = {held[k][0], held[k][1], held[k][2], held[k][3]};
+    for (int k = 0; k < STATE_HELD; k += STATE_CHUNKS) {
+      if (threadIdx.x + (k + STATE_CHUNKS - 1) * THREADS < chunks) {
+        float e[4 * STATE_CHUNKS];
+#pragma unroll
+        for (int q = 0; q < 4 * STATE_CHUNKS; ++q) e[q] = held[k + q / 4][q % 4];
         add_values<true>(t, e, evidence);
+      } else {
+#pragma unroll
+        for (int j = k; j < k + STATE_CHUNKS; ++j) {
+          if (threadIdx.x + j * THREADS < chunks) {
+            const float e[4] = {held[j][0], held[j][1], held[j][2], held[j][3]};
+            add_values<true>(t, e, evidence);
+          }
+        }
       }
     }
-    add_chunks<true>(t, x, STATE_HELD * STATE_THREADS, chunks, evidence);
-    add_tail<true>(t, x, vocab, evidence);
-    t = block_stats(t);
+    add_chunks<THREADS, true>(t, x, STATE_HELD * THREADS, chunks, evidence);
+    add_tail<THREADS, true>(t, x, vocab, evidence);
+    t = block_stats<THREADS>(t);
   }
   const DivBy div(t.s * EXP_SCALE);
   auto put = [&](int64_t c, f32x4_t v) {
@@ -384,14 +400,14 @@ __global__ __launch_bounds__(STATE_THREADS) void state_embed_rows_kernel(const f
   if constexpr (POST) {
     if (part.first == 0) {
 #pragma unroll
-      for (int k = 0; k < STATE_HELD; ++k, c += STATE_THREADS)
+      for (int k = 0; k < STATE_HELD; ++k, c += THREADS)
         if (c < part.end) put(c, held[k]);
     }
   }
 #pragma unroll 4
-  for (; c < part.end; c += STATE_THREADS) put(c, load_last<NT>(x + 4 * c));
+  for (; c < part.end; c += THREADS) put(c, load_last<NT>(x + 4 * c));
   if (!part.last) return;
-  for (int64_t i = 4 * chunks + threadIdx.x; i < vocab; i += STATE_THREADS) {
+  for (int64_t i = 4 * chunks + threadIdx.x; i < vocab; i += THREADS) {
     if constexpr (POST)
       post[i] = (uint16_t)(pack_bf16x2(div(exp_scaled(below<true>(x[i], evidence, t.m))), 0.f) & 0xffffu);
     raw[i] = (uint16_t)(pack_bf16x2(x[i], 0.f) & 0xffffu);
@@ -399,8 +415,8 @@ __global__ __launch_bounds__(STATE_THREADS) void state_embed_rows_kernel(const f
 }
 
 // state[r] = (c_keep * state[r] + c_new * softmax(logits[r])) / c_div in place, logits bf16.
-template <bool NT>
-__global__ __launch_bounds__(STATE_THREADS) void state_update_kernel(float *__restrict__ state, int64_t vocab,
+template <bool NT, int THREADS>
+__global__ __launch_bounds__(THREADS) void state_update_kernel(float *__restrict__ state, int64_t vocab,
                                                                      int64_t ss, const uint16_t *__restrict__ logits,
                                                                      int64_t ls, float c_keep, float c_new,
                                                                      float c_div) {
@@ -410,15 +426,15 @@ __global__ __launch_bounds__(STATE_THREADS) void state_update_kernel(float *__re
   const int64_t chunks = vocab >> 2;
   const PartOf part = part_of(chunks);
   RowStats t = RowStats::none();
-  add_chunks<false>(t, lg, 0, chunks, 1.f);
-  add_tail<false>(t, lg, vocab, 1.f);
-  t = block_stats(t);
+  add_chunks<THREADS, false>(t, lg, 0, chunks, 1.f);
+  add_tail<THREADS, false>(t, lg, vocab, 1.f);
+  t = block_stats<THREADS>(t);
   const DivBy div(t.s * EXP_SCALE), scale(c_div);
   auto upd = [&](float s, float l) {
     return scale.any(__builtin_fmaf(c_keep, s, c_new * div(exp_scaled(l - t.m))));
   };
 #pragma unroll 4
-  for (int64_t c = part.first + threadIdx.x; c < part.end; c += STATE_THREADS) {
+  for (int64_t c = part.first + threadIdx.x; c < part.end; c += THREADS) {
     const int64_t at = 4 * c;
     const f32x4_t l = load4(lg + at);
     f32x4_t v = load_last<NT>(x + at);
@@ -427,7 +443,7 @@ __global__ __launch_bounds__(STATE_THREADS) void state_update_kernel(float *__re
     store_last<NT>(x + at, v);
   }
   if (!part.last) return;
-  for (int64_t i = 4 * chunks + threadIdx.x; i < vocab; i += STATE_THREADS) x[i] = upd(x[i], load1(lg + i));
+  for (int64_t i = 4 * chunks + threadIdx.x; i < vocab; i += THREADS) x[i] = upd(x[i], load1(lg + i));
 }
 
 // Whether a call's state rows outgrow the 256 MB of the last cache level. Below that the
@@ -435,16 +451,26 @@ __global__ __launch_bounds__(STATE_THREADS) void state_update_kernel(float *__re
 // accesses only cost: the state rows alone at 256 x 151936 (156 MB) 33 us, 42 us with them.
 static bool state_streams(int64_t rows, int64_t vocab) { return rows * vocab > (64ll << 20); }
 
-// Workgroups per row, a power of two: with fewer rows than two per CU the rest of the chip
-// takes parts of them, each part reading the whole row for its statistics again (from the
-// caches).
+// Workgroups per row, a power of two: doubled while they are no more than the CUs (so 257 rows
+// and more are not split on 256 CUs); each part reads the whole row for its statistics again
+// (from the caches).
 static unsigned state_parts(int64_t rows) {
   DeviceInfo info;
   if (device_info(&info) != FM_OK) return 1;
   unsigned p = 1;
-  while (p < 8 && 2 * p * rows <= 2 * (int64_t)info.cus) p *= 2;
+  while (p < 8 && p * rows <= (int64_t)info.cus) p *= 2;
   return p;
 }
+
+// Threads per workgroup, by the vocabulary alone (so that the order of a row's sum is). Short
+// rows want small workgroups: what a row costs is then its barrier and its one round of loads.
+// us, 256 / 512 / 1024 threads, update and embedding: 8192 x 1000 22 / 39 / 95 and 20 / 40 /
+// 106; 1024 x 8192 15 / 17 / 23 and 17 / 17 / 24; 1024 x 16384 30 / 30 / 33 and 26 / 27 / 35;
+// 1024 x 32000 58 / 58 / 59 and 54 / 50 / 55; 300 x 65536 47 / 45 / 49 and 41 / 44 / 48; 1024
+// x 65536 143 / 139 / 136 and 146 / 145 / 127; 1024 x 151936 333 / 321 / 283 and 309 / 289 /
+// 260. (Every size with 256 threads, expf and IEEE divisions: 32 and 30, 21 and 18, 38 and 33,
+// 71 and 61, 86 and 75, 173 and 164, 422 and 388.)
+static int state_threads(int64_t vocab) { return vocab <= 12288 ? 256 : vocab <= 40960 ? 512 : 1024; }
 
 }  // namespace fm
 
@@ -533,12 +559,29 @@ extern "C" int fm_state_embed_rows(const float *state, int64_t rows, int64_t voc
              "state must be 16-byte aligned with a row stride that is a multiple of 4 covering a row");
   FM_REQUIRE(((uintptr_t)out & 7) == 0 && out_stride % 4 == 0 && out_stride >= vocab,
              "out must be 8-byte aligned with a row stride that is a multiple of 4 covering a row");
-  const dim3 grid((unsigned)rows, posterior ? state_parts(rows) : 1u), block(STATE_THREADS);
   const bool nt = state_streams(rows, vocab);
-  auto *kernel = posterior ? (nt ? state_embed_rows_kernel<true, true> : state_embed_rows_kernel<true, false>)
-                           : (nt ? state_embed_rows_kernel<false, true> : state_embed_rows_kernel<false, false>);
-  kernel<<<grid, block, 0, (hipStream_t)stream>>>(state, vocab, state_stride, evidence, (uint16_t *)out, out_stride,
-                                                  rows);
+  auto run = [&](auto *kernel, int threads, unsigned parts) {
+    kernel<<<dim3((unsigned)rows, parts), dim3(threads), 0, (hipStream_t)stream>>>(
+        state, vocab, state_stride, evidence, (uint16_t *)out, out_stride, rows);
+  };
+#define FM_EMBED(THREADS) \
+  run(nt ? state_embed_rows_kernel<true, true, THREADS> : state_embed_rows_kernel<true, false, THREADS>, THREADS, parts)
+  const int threads = state_threads(vocab);
+  const unsigned parts = state_parts(rows);
+  // The state rows alone are a copy: 1024 threads where they stream (1024 x 151936 171 us, 175
+  // with 256), 256 below (300 x 151936 54 us, 57 with 1024; 8192 x 1000 8.2 and 11.2 us), in
+  // half as many parts (256 x 151936 33.9 us, 34.9 in two).
+  if (!posterior && nt)
+    run(state_embed_rows_kernel<false, true, 1024>, 1024, 1);
+  else if (!posterior)
+    run(state_embed_rows_kernel<false, false, 256>, 256, state_parts(2 * rows));
+  else if (threads == 256)
+    FM_EMBED(256);
+  else if (threads == 512)
+    FM_EMBED(512);
+  else
+    FM_EMBED(1024);
+#undef FM_EMBED
   FM_CHECK_HIP(hipGetLastError());
   return FM_OK;
 }
@@ -558,9 +601,20 @@ extern "C" int fm_state_update(float *state, int64_t rows, int64_t vocab, int64_
   // The scalars as torch takes Python floats into a float32 op: computed in double, then
   // rounded to float.
   const float c_keep = (float)(1.0 - end), c_new = (float)(end - start), c_div = (float)(1.0 - start);
-  auto *kernel = state_streams(rows, vocab) ? state_update_kernel<true> : state_update_kernel<false>;
-  kernel<<<dim3((unsigned)rows, state_parts(rows)), dim3(STATE_THREADS), 0, (hipStream_t)stream>>>(
-      state, vocab, state_stride, (const uint16_t *)logits, logits_stride, c_keep, c_new, c_div);
+  const bool nt = state_streams(rows, vocab);
+  auto run = [&](auto *kernel, int threads) {
+    kernel<<<dim3((unsigned)rows, state_parts(rows)), dim3(threads), 0, (hipStream_t)stream>>>(
+        state, vocab, state_stride, (const uint16_t *)logits, logits_stride, c_keep, c_new, c_div);
+  };
+#define FM_UPDATE(THREADS) run(nt ? state_update_kernel<true, THREADS> : state_update_kernel<false, THREADS>, THREADS)
+  const int threads = state_threads(vocab);
+  if (threads == 256)
+    FM_UPDATE(256);
+  else if (threads == 512)
+    FM_UPDATE(512);
+  else
+    FM_UPDATE(1024);
+#undef FM_UPDATE
   FM_CHECK_HIP(hipGetLastError());
   return FM_OK;
 }

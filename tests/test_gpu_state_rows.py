@@ -108,9 +108,9 @@ def test_subnormal_probabilities(dev):
     assert ((out - 0.5 * d64).abs() <= 2.0 ** -148 + 1e-6 * d64).all()
 
 
-@pytest.mark.parametrize("vocab", [1003, 32770, 49157, 151936])
+@pytest.mark.parametrize("vocab", [1003, 16385, 32770, 49157, 151936])
 def test_rows_do_not_depend_on_the_others(dev, vocab):
-    """A row's values bit for bit, whether the call has 1, 16, 64, 200 or 300 rows (eight to
+    """A row's values bit for bit, whether the call has 1, 16, 64, 100 or 300 rows (eight to
     one workgroups a row)."""
     print(f"state rows alone and together vocab={vocab}", flush=True)
     g = torch.Generator(device=dev).manual_seed(vocab)
@@ -118,7 +118,7 @@ def test_rows_do_not_depend_on_the_others(dev, vocab):
     logits = _rows(2 * torch.randn(300, vocab, generator=g, device=dev, dtype=torch.bfloat16), dev)
     whole = ops.state_embed_rows(state, 3.0)
     moved = ops.state_update(_rows(state, dev), logits, 0.2, 0.7)
-    for rows in (1, 16, 64, 200):
+    for rows in (1, 16, 64, 100):
         part = ops.state_embed_rows(state[:rows], 3.0)
         assert torch.equal(part[:rows], whole[:rows]), (rows, "posterior")
         assert torch.equal(part[rows:], whole[300:300 + rows]), (rows, "state")
@@ -152,11 +152,17 @@ def test_state_wrapper_checks(dev):
         ops.state_update(torch.zeros(2, 8, device=dev), torch.zeros(2, 8, device=dev), 0.0, 0.5)
 
 
-# rows: 1 and 3 take eight workgroups a row, 200 two, 300 one; vocab: less than a chunk per
-# thread, around the 32768 values a workgroup keeps in registers and the chunks of a step,
-# remainders of 1 to 3; the last case is past the size whose accesses are non-temporal.
-@pytest.mark.parametrize("rows,vocab", [(r, v) for r in (1, 3, 200, 300)
-                                        for v in (1, 5, 4099, 32767, 32770, 49156)] + [(520, 131075)])
+# rows: 1 and 3 take eight workgroups a row, 64 four, 100 and 128 two, 200 and 300 one; vocab:
+# less than a chunk per thread, both sides of the lines between 256, 512 and 1024 threads, around
+# what a workgroup keeps in registers (32 values a thread) and the chunks of a step, remainders
+# of 1 to 3; (64, 151936) and (100, 131075) read parts of split rows again; the last ones are past
+# the size whose accesses are non-temporal, at 1024, 512 and 256 threads.
+_EDGES = [(r, v) for r in (1, 3, 128, 200, 300)
+          for v in (1, 5, 4099, 8193, 12288, 12291, 32767, 32770, 40960, 40961, 49156)]
+_EDGES += [(64, 151936), (100, 131075), (520, 131075), (2100, 32001), (16500, 4099)]
+
+
+@pytest.mark.parametrize("rows,vocab", _EDGES)
 def test_state_kernels_edges(dev, rows, vocab):
     """Masked values (-inf, the lowest finite value), +inf and NaN as torch's softmax takes
     them, and the sizes where a row's workgroups and passes change."""
@@ -180,6 +186,8 @@ def test_state_kernels_edges(dev, rows, vocab):
     # 2^-133 below its normal range
     assert torch.allclose(both[:rows].double(), post, rtol=2.0 ** -8, atol=2.0 ** -133, equal_nan=True)
     assert torch.equal(both[rows:].view(torch.int16), state.bfloat16().view(torch.int16))
+    alone = ops.state_embed_rows(state, 1.5, posterior=False)
+    assert torch.equal(alone.view(torch.int16), state.bfloat16().view(torch.int16))
     want = (0.4 * before + 0.3 * torch.softmax(logits.double(), -1)) / 0.7
     out = ops.state_update(state, logits, 0.3, 0.6).double()
     big = want.abs() > 1e38  # beyond float32 on the way to the quotient
