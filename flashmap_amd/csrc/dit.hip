@@ -341,7 +341,7 @@ __device__ __forceinline__ PartOf part_of(int64_t chunks) {
   return PartOf{chunks * p >> sh, chunks * (p + 1) >> sh, p == parts - 1};
 }
 
-// POST: rows r < rows of out get bf16(softmax(evidence * state[r])) and rows rows + r
+// POST: rows r < rows of out (`rows`: the call's, where out begins at this launch's) get bf16(softmax(evidence * state[r])) and rows rows + r
 // bf16(state[r]); otherwise out holds the state rows only (one read of the row). A
 // workgroup keeps the row's first STATE_HELD chunks per thread in registers between the two
 // passes (32768 values of 1024 threads), for the part that begins there; the rest is read
@@ -472,6 +472,13 @@ static unsigned state_parts(int64_t rows) {
 // 71 and 61, 86 and 75, 173 and 164, 422 and 388.)
 static int state_threads(int64_t vocab) { return vocab <= 12288 ? 256 : vocab <= 40960 ? 512 : 1024; }
 
+// launch(first row, rows) over slices of a call's rows: a grid counts at most 2^32 - 1 threads.
+template <typename F>
+static void for_row_slices(int64_t rows, F &&launch) {
+  constexpr int64_t SLICE = 1 << 20;
+  for (int64_t r = 0; r < rows; r += SLICE) launch(r, (unsigned)(rows - r < SLICE ? rows - r : SLICE));
+}
+
 }  // namespace fm
 
 extern "C" int fm_adaln_residual(const void *x, int64_t x_stride, const void *y, int64_t y_stride,
@@ -561,8 +568,11 @@ extern "C" int fm_state_embed_rows(const float *state, int64_t rows, int64_t voc
              "out must be 8-byte aligned with a row stride that is a multiple of 4 covering a row");
   const bool nt = state_streams(rows, vocab);
   auto run = [&](auto *kernel, int threads, unsigned parts) {
-    kernel<<<dim3((unsigned)rows, parts), dim3(threads), 0, (hipStream_t)stream>>>(
-        state, vocab, state_stride, evidence, (uint16_t *)out, out_stride, rows);
+    for_row_slices(rows, [&](int64_t first, unsigned n) {
+      kernel<<<dim3(n, parts), dim3(threads), 0, (hipStream_t)stream>>>(
+          state + first * state_stride, vocab, state_stride, evidence, (uint16_t *)out + first * out_stride,
+          out_stride, rows);
+    });
   };
 #define FM_EMBED(THREADS) \
   run(nt ? state_embed_rows_kernel<true, true, THREADS> : state_embed_rows_kernel<true, false, THREADS>, THREADS, parts)
@@ -602,9 +612,13 @@ extern "C" int fm_state_update(float *state, int64_t rows, int64_t vocab, int64_
   // rounded to float.
   const float c_keep = (float)(1.0 - end), c_new = (float)(end - start), c_div = (float)(1.0 - start);
   const bool nt = state_streams(rows, vocab);
+  const unsigned parts = state_parts(rows);
   auto run = [&](auto *kernel, int threads) {
-    kernel<<<dim3((unsigned)rows, state_parts(rows)), dim3(threads), 0, (hipStream_t)stream>>>(
-        state, vocab, state_stride, (const uint16_t *)logits, logits_stride, c_keep, c_new, c_div);
+    for_row_slices(rows, [&](int64_t first, unsigned n) {
+      kernel<<<dim3(n, parts), dim3(threads), 0, (hipStream_t)stream>>>(
+          state + first * state_stride, vocab, state_stride, (const uint16_t *)logits + first * logits_stride,
+          logits_stride, c_keep, c_new, c_div);
+    });
   };
 #define FM_UPDATE(THREADS) run(nt ? state_update_kernel<true, THREADS> : state_update_kernel<false, THREADS>, THREADS)
   const int threads = state_threads(vocab);

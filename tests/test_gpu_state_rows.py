@@ -194,3 +194,20 @@ def test_state_kernels_edges(dev, rows, vocab):
     assert torch.allclose(torch.where(big, 0.0, out), torch.where(big, 0.0, want), rtol=2e-5, atol=2e-6,
                           equal_nan=True)
     assert torch.equal(out[big].sign(), want[big].sign())
+
+
+def test_more_rows_than_a_grid_counts_threads_for(dev):
+    """Short rows by the million: 2^22 + 5 workgroups of 1024 threads were past the 2^32 threads
+    that a launch counts, and the last rows stayed unwritten, with no error."""
+    rows, vocab = (1 << 22) + 5, 3
+    g = torch.Generator(device=dev).manual_seed(5)
+    state = _rows(torch.randn(rows, vocab, generator=g, device=dev), dev)
+    logits = _rows(torch.randn(rows, vocab, generator=g, device=dev, dtype=torch.bfloat16), dev)
+    both = ops.state_embed_rows(state, 1.5)
+    post = torch.softmax(1.5 * state.double(), -1)
+    assert torch.allclose(both[:rows].double(), post, rtol=2.0 ** -8, atol=0)
+    assert torch.equal(both[rows:], state.bfloat16())
+    assert torch.equal(ops.state_embed_rows(state, 1.5, posterior=False), state.bfloat16())
+    want = (0.4 * state.double() + 0.3 * torch.softmax(logits.double(), -1)) / 0.7
+    out = ops.state_update(state, logits, 0.3, 0.6).double()
+    assert torch.allclose(out, want, rtol=2e-6, atol=1e-6)
