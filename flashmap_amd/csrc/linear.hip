@@ -102,6 +102,8 @@ extern "C" int fm_linear_rows(const void *x, int64_t x_stride, const void *weigh
   if (rows == 0 || n == 0) return FM_OK;
   if (rows > 32 || k % 32 != 0)
     return fail(FM_ERR_UNSUPPORTED, "%d rows of %d: at most 32 rows, a multiple of 32 values", rows, k);
+  if (n > 1 << 26)  // a launch counts at most 2^32 threads
+    return fail(FM_ERR_UNSUPPORTED, "%d output columns: at most 2^26", n);
   FM_REQUIRE(x && weight && out, "NULL tensor pointer");
   FM_REQUIRE((((uintptr_t)x | (uintptr_t)weight) & 15) == 0, "x / weight must be 16-byte aligned");
   FM_REQUIRE(x_stride % 8 == 0 && w_stride % 8 == 0 && x_stride >= k && w_stride >= k && out_stride >= n,

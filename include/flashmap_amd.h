@@ -435,7 +435,7 @@ int fm_adaln_residual(const void *x, int64_t x_stride, const void *y, int64_t y_
  * flashmap/modeling_flashmap.py:118-192): out = x weight^T (+ bias in fp32), rounded to
  * bf16 once. x (rows, k), weight (n, k), bias (n,) or NULL, out (rows, n), all bf16 with
  * row strides in elements (x, weight: 16-byte aligned, strides multiples of 8). rows at
- * most 32, k a multiple of 32. */
+ * most 32, n at most 2^26, k a multiple of 32. */
 int fm_linear_rows(const void *x, int64_t x_stride, const void *weight, int64_t w_stride,
                    const void *bias, void *out, int64_t out_stride, int32_t rows, int32_t n,
                    int32_t k, void *stream);

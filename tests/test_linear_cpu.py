@@ -9,7 +9,7 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
-from flashmap_amd import drafter, ops
+from flashmap_amd import _native, drafter, ops
 
 
 def test_cpu_calls_are_torchs():
@@ -104,3 +104,13 @@ def test_what_was_put_around_a_projection_runs():
         handle.remove()
     assert drafter._bare(plain)
     assert torch.equal(drafter._project(replaced, torch.ones(2)), torch.ones(2))
+
+
+def test_entry_refuses_what_it_cannot_launch():
+    """The C entry's own checks, which return before anything is launched."""
+    at = 4096  # an aligned address that no check follows
+    for rows, n, k in ((33, 16, 64), (16, 16, 48), (16, (1 << 26) + 1, 64)):
+        with pytest.raises(_native.NativeError, match="at most"):
+            ops.call("fm_linear_rows", at, k, at, k, None, at, n, rows, n, k, None)
+    with pytest.raises(_native.NativeError, match="aligned"):
+        ops.call("fm_linear_rows", at + 2, 64, at, 64, None, at, 16, 16, 16, 64, None)
