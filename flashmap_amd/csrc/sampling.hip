@@ -189,8 +189,8 @@ __global__ __launch_bounds__(SEL_THREADS) void select_tiles_kernel(const SelectA
 // workgroup has seen (an LDS maximum that only rises; a late read of it only costs work). A
 // wavefront first draws for its 64 lanes' largest logits of the tile, which sets the
 // bound near the tile's best at once, then for the rest that pass it, gathered from the
-// lanes into an LDS queue and taken 64 at a time; where most pass (flat logits), each lane
-// takes its own instead, read again from the caches. The uniform word alone rules most
+// lanes into an LDS queue and taken 64 at a time; where most of a single tile pass (flat
+// logits), each lane takes its own instead, read again from the caches. The uniform word alone rules most
 // of these out before the logarithms. Keys, and so tokens, are those of every logit's own
 // noise: what is skipped is below the maximum by more than the bound's rounding. The bound
 // is no bound (-inf: nothing is skipped) for temperatures whose product with it could over-
@@ -198,15 +198,17 @@ __global__ __launch_bounds__(SEL_THREADS) void select_tiles_kernel(const SelectA
 //
 // How much is left depends on the logits and T: of 151936 normal logits with 24 likely ones
 // 1 % to 30 % for T from 0.6 to 1.2. Measured on 1024 x 151936 bf16, us (every logit drawn for
-// / this kernel): half the rows greedy, T of 0.6 to 1.2: 209 / 125; all sampled at 0.6 340 /
-// 83, 1.2 340 / 202; normal logits of sigma 1 331 / 329, equal logits 330 / 329; all greedy
-// 75 / 54. Rows that are not 16-byte aligned are read in whole granules all the same (RowView):
-// 1024 x 100003 half greedy 184 (logit by logit) / 89, all greedy 122 / 44.
+// / this kernel): half the rows greedy, T of 0.6 to 1.2: 209 / 111; all sampled at 0.6 330 /
+// 69, 1.2 330 / 189; normal logits of sigma 1 327 / 306, equal logits 328 / 314; all greedy
+// 74 / 54. Rows that are not 16-byte aligned are read in whole granules all the same (RowView):
+// 1024 x 99999 half greedy 181 (logit by logit) / 82, all greedy 121 / 42.
 constexpr float GUMBEL_MAX = 16.64f;
 constexpr int SAMPLE_IT = 4;  // 8-logit chunks per thread of a tile
 constexpr int sample_tile(int threads) { return 8 * SAMPLE_IT * threads; }
-// More than this many of a wavefront's first 512 logits of a tile above the bound: past the
-// queue. 1024 x 151936, T = 1.2: 267 us at 256, 250 at 400, 252 without; equal logits 318, 318, 338.
+// More than this many of a wavefront's first 512 logits above the bound: past the queue (for
+// workgroups of one tile; over several the queue has more to gather and the choice costs more
+// than it gives: 1024 x 151936, T = 1.2, 1024 threads 189 us, 208 with it). 1024 x 151936 in
+// single tiles, T = 1.2: 267 us at 256, 250 at 400, 252 without; equal logits 318, 318, 338.
 constexpr int SAMPLE_DIRECT = 400;
 constexpr int SAMPLE_QUEUE = 64 + 4 * 64;  // what a drain leaves and four logits of 64 lanes
 
@@ -468,9 +470,14 @@ __global__ __launch_bounds__(THREADS, TY == LOGITS_F32 ? 4 : 8) void sample_part
     bool take = true;
     if (SEVERAL && g != first) {
       lower();
-      bool nan;
-      const float m = tile_max<TY>(x, nan);
-      take = __ballot(!(m < low) || nan) != 0;
+      bool any = false;
+#pragma unroll
+      for (int it = 0; it < SAMPLE_IT; ++it) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) any |= !(x[it].at(j) < low);
+        x[it].forget();
+      }
+      take = __ballot(any) != 0;
     }
     if (take) {
       float top = x[0].at(0);
@@ -489,10 +496,12 @@ __global__ __launch_bounds__(THREADS, TY == LOGITS_F32 ? 4 : 8) void sample_part
       if (g == first) __syncthreads();        // every wavefront's, before any logit is taken
       lower();
       int likely = 0;  // of 512 logits
+      if constexpr (!SEVERAL) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) likely += __popcll(__ballot(!(x[0].at(j) < low)));
-      x[0].forget();
-      if (likely > SAMPLE_DIRECT) {  // most can win: each lane takes its own, without the queue
+        for (int j = 0; j < 8; ++j) likely += __popcll(__ballot(!(x[0].at(j) < low)));
+        x[0].forget();
+      }
+      if (!SEVERAL && likely > SAMPLE_DIRECT) {  // most can win: each lane takes its own, without the queue
 #pragma unroll 1
         for (uint32_t h = g; h < g + CHUNKS && h < chunks; h += THREADS) {
           if (h + threadIdx.x < chunks) {
@@ -514,7 +523,7 @@ __global__ __launch_bounds__(THREADS, TY == LOGITS_F32 ? 4 : 8) void sample_part
               }
             }
           }
-          if (SEVERAL || h + THREADS < chunks) {
+          if (h + THREADS < chunks) {
             raise(bk);
             lower();
           }
@@ -610,9 +619,9 @@ struct SamplePlan {
   int64_t parts;
 };
 // Logits from which a call's workgroups carry their bound over several tiles. Below, one
-// 256-thread tile each spreads best; us, 256 threads / 512 threads over two tiles, 304 x
-// 151936: T = 0.6 45 / -, 400 x 151936 (above): T = 0.6 56 / 48, 1.2 112 / 111, half greedy
-// 63 / 67, equal 131 / 139; 640 x 151936 79 / 66, 170 / 160, 94 / 90, 201 / 212.
+// 256-thread tile each spreads best; us, 256 threads / 512 threads over two tiles, 400 x
+// 151936 (above): T = 0.6 56 / 47, 1.2 112 / 105, half greedy 63 / 63, equal 131 / 140; 640 x
+// 151936 79 / 63, 170 / 151, 94 / 89, 201 / 210.
 constexpr int64_t SAMPLE_LARGE = 50 << 20;
 // Rows of at most 2048 columns: one wavefront each from here on, below 256 threads that draw
 // for every logit (sample_short). 8192 x 1000: T = 0.6 18 us, equal logits 34 (36 with 256
@@ -626,9 +635,10 @@ static int64_t sample_span(int64_t vocab, bool vec) { return vec ? vocab : vocab
 // Large calls on 2-byte logits: one 1024-thread workgroup per row, whose bound is the row's
 // own, where the rows fill the CUs evenly (the last round of rows at least 95 % full);
 // elsewhere the CUs with a row more would set the time (640 x 151936, equal logits: 251 us
-// against 212), and 512 threads take two tiles each. us, 1024 x 151936, 1024 threads / 512:
-// T = 0.6 76 / 98, 1.2 202 / 243, half greedy 138 / 129, equal 333 / 327. Float32 tiles leave
-// room for half the wavefronts there (equal logits 390 us against 321 with 256 threads).
+// against 210), and 512 threads take two tiles each. us, 1024 x 151936, 1024 threads / 512:
+// T = 0.6 76 / 98, 1.2 202 / 243, half greedy 138 / 129, equal 333 / 327 (before the last
+// shortening of both). Float32 tiles leave room for half the wavefronts there (equal logits
+// 390 us against 321 with 256 threads).
 static SamplePlan sample_plan(int64_t rows, int64_t vocab, bool vec, bool half) {
   const int64_t span = sample_span(vocab, vec);
   auto tiles = [&](int threads) { return (span + sample_tile(threads) - 1) / sample_tile(threads); };
