@@ -167,7 +167,8 @@ def _project(module: nn.Module, x: torch.Tensor) -> torch.Tensor:
         return module(x)
     if x.dim() == 0 or x.numel() > ops.LINEAR_ROWS * x.shape[-1] or not _bare(module):
         return module(x)
-    y = ops.linear_rows(x, module.weight, module.bias)
+    held = module._parameters  # past nn.Module's attribute lookup
+    y = ops._few_rows(x, held["weight"], held["bias"])
     return module(x) if y is None else y
 
 
@@ -223,7 +224,7 @@ class FlashMapAdaLayerNorm(nn.Module):
 
     def modulation(self, cond: torch.Tensor):
         """``(scale, shift, gate)`` of the conditioning ``cond``."""
-        return self.linear(F.silu(cond)).chunk(3, dim=-1)
+        return _project(self.linear, F.silu(cond)).chunk(3, dim=-1)
 
     def forward(self, x: torch.Tensor, modulation):
         scale, shift, gate = modulation

@@ -1229,31 +1229,32 @@ def _linear_streams(rows: int, n: int, k: int) -> bool:
 def _followed() -> bool:
     """Whether a compiler or tracer follows the call (torch.compile, torch.export, jit.trace;
     a symbolic tracer's values show by their type)."""
-    return torch.compiler.is_compiling() or torch.jit.is_tracing()
+    return torch.compiler.is_compiling() or torch._C._is_tracing()
 
 
-def _eager_here(*tensors: torch.Tensor | None) -> bool:
-    """Whether a plain kernel launch is all that a call on these tensors asks for: CUDA
-    tensors, no gradient (backward or forward mode), and nothing that watches or rewrites
-    torch's calls (autocast, subclasses and modes, functorch's transforms)."""
-    given = [t for t in tensors if t is not None]
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def _eager_here(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> bool:
+    """Whether a plain kernel launch is all that a call on these tensors asks for: no
+    gradient (backward or forward mode), and nothing that watches or rewrites torch's calls
+    (autocast, subclasses and modes, functorch's transforms)."""
     return (
-        all(t.is_cuda and type(t) in (torch.Tensor, torch.nn.Parameter) for t in given)
-        and not (torch.is_grad_enabled() and any(t.requires_grad for t in given))
+        type(weight) in _PLAIN
+        and (bias is None or type(bias) in _PLAIN)
+        and not (torch.is_grad_enabled()
+                 and (x.requires_grad or weight.requires_grad or (bias is not None and bias.requires_grad)))
         and not torch.is_autocast_enabled("cuda")
-        and not torch.overrides.has_torch_function(given)
+        and not torch.overrides.has_torch_function((x, weight))
         and torch._C._len_torch_dispatch_stack() == 0
         and torch._C._functorch.peek_interpreter_stack() is None
         and torch.autograd.forward_ad._current_level < 0
     )
 
 
-def linear_rows(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor | None:
-    """``F.linear`` of few bf16 rows, which only stream the weights (``_linear_streams``), by
-    fm_linear_rows; None for every other call and for those that ask for more than a launch
-    (``_eager_here``). What a compiler or tracer follows is decided first, before anything
-    of ``x`` is looked at: their graphs hold torch's Linear alone."""
-    if _followed() or type(x) is not torch.Tensor or not x.is_cuda or weight.dim() != 2:
+def _few_rows(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> torch.Tensor | None:
+    """:func:`linear_rows` of a CUDA tensor that no compiler or tracer follows."""
+    if weight.dim() != 2:
         return None
     n, k = weight.shape
     if x.numel() > LINEAR_ROWS * k:  # most calls: no further looks
@@ -1263,15 +1264,21 @@ def linear_rows(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None
         rows > 0
         and _linear_streams(rows, n, k)
         and x.shape[-1] == k
-        and x.dtype == weight.dtype == torch.bfloat16
-        and (bias is None or (bias.dtype == torch.bfloat16 and bias.is_contiguous() and bias.shape == weight.shape[:1]))
+        and x.dtype is torch.bfloat16
+        and weight.dtype is torch.bfloat16
+        and (bias is None or (bias.dtype is torch.bfloat16 and bias.dim() == 1 and bias.numel() == n
+                              and bias.is_contiguous()))
         and x.is_contiguous()
         and weight.stride(1) == 1
         and weight.stride(0) % 8 == 0
         and weight.stride(0) >= k
         and _eager_here(x, weight, bias)
-        and x.device == weight.device == (x.device if bias is None else bias.device)
-        and x.device.index == torch.cuda.current_device()
+    ):
+        return None
+    device = x.get_device()
+    if not (
+        device == weight.get_device() == torch.cuda.current_device()
+        and (bias is None or device == bias.get_device())
         and x.data_ptr() % 16 == 0
         and weight.data_ptr() % 16 == 0
     ):
@@ -1280,6 +1287,16 @@ def linear_rows(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None
     call("fm_linear_rows", x.data_ptr(), k, weight.data_ptr(), weight.stride(0), _ptr(bias), out.data_ptr(), n,
          rows, n, k, _stream(x))
     return out
+
+
+def linear_rows(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor | None:
+    """``F.linear`` of few bf16 rows, which only stream the weights (``_linear_streams``), by
+    fm_linear_rows; None for every other call and for those that ask for more than a launch
+    (``_eager_here``). What a compiler or tracer follows is decided first, before anything
+    of ``x`` is looked at: their graphs hold torch's Linear alone."""
+    if _followed() or type(x) is not torch.Tensor or not x.is_cuda:
+        return None
+    return _few_rows(x, weight, bias)
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
