@@ -168,7 +168,10 @@ def _project(module: nn.Module, x: torch.Tensor) -> torch.Tensor:
     if x.dim() == 0 or x.numel() > ops.LINEAR_ROWS * x.shape[-1] or not _bare(module):
         return module(x)
     held = module._parameters  # past nn.Module's attribute lookup
-    y = ops._few_rows(x, held["weight"], held["bias"])
+    weight = held.get("weight")
+    if weight is None or "bias" not in held:  # set as plain attributes
+        return module(x)
+    y = ops._few_rows(x, weight, held["bias"])
     return module(x) if y is None else y
 
 

@@ -115,6 +115,14 @@ def test_modules_take_the_kernel_and_keep_their_hooks(dev, launches):
         assert torch.equal(torch.compile(mlp, fullgraph=True, backend="eager")(x), want)
         assert torch.equal(torch.jit.trace(mlp, x, check_trace=False)(x), want)
         assert launches == []
+        plain = drafter.FlashMapMLP(cfg).bfloat16().to(dev)
+        plain.load_state_dict(mlp.state_dict())
+        weight = plain.fc1.weight.detach()
+        del plain.fc1.weight
+        plain.fc1.weight = weight  # no parameter any more
+        launches.clear()
+        assert plain(x).shape == want.shape and launches == ["fm_linear_rows"]  # fc2's
+        launches.clear()
         seen = []
         mlp.fc1.register_forward_hook(lambda m, args, out: seen.append(out))
         hooked = mlp(x)
