@@ -385,7 +385,8 @@ int fm_write_context_kv_pool_fp8(const void *kv, int64_t tokens, int32_t layers,
  * f3: the draft step's token selection and noise. Logits are (rows, vocab) with
  * row_stride elements between rows, dtype 0 bf16, 1 fp16, 2 fp32; out is int64 (rows,).
  * The selection calls use a caller workspace of fm_select_workspace_bytes(rows, vocab)
- * bytes. The random stream is Triton's tl.rand / tl.randn (Philox-4x32-10 keyed by the
+ * bytes. The sampler reads rows in whole 16-byte granules, those with a logit of the row in
+ * them. The random stream is Triton's tl.rand / tl.randn (Philox-4x32-10 keyed by the
  * seed's words, counter (offset, 0, 0, 0)) word for word.
  */
 size_t fm_select_workspace_bytes(int64_t rows, int64_t vocab);
